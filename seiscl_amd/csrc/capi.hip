@@ -101,6 +101,19 @@ struct seis_ctx {
         size_t cap;
         hipEvent_t freed;           // compute-stream point after the last use
     };
+    // workspace of resident 2D runs (fd2d_resident.hip): exchange words and the
+    // run's counters, a host word that a run which gave up sets.  One run at a time uses it (mu).
+    struct Resident {
+        std::mutex mu;
+        void *words = nullptr;
+        size_t bytes = 0;
+        int *failed = nullptr;      // pinned host memory
+        // CUs; 0: no resident runs (no cooperative launch, or a run gave up:
+        // the GPU is shared with another program's kernels)
+        int ncu = 0;
+        // longest wait of a block for another, in wall_clock64 ticks
+        long long patience = 0;
+    } resident;
     std::map<void *, size_t> allocs;          // live block -> requested bytes
     std::map<void *, size_t> caps;            // every block -> capacity
     std::multimap<size_t, std::pair<void *, hipEvent_t>> cache;   // released blocks
@@ -628,6 +641,138 @@ void step_all(seis_model *m, int t, hipStream_t st, const int *tb = nullptr) {
     if (m->c.freesurf && !m->a.fuse_surface) step_surface(m, st);
 }
 
+// ---- 2D runs resident on the chip (fd2d_resident.hip) -----------------------
+// Runs shorter than this stay with the step kernels: the launch, the loading of
+// the tiles and the final agreement of the blocks cost about as much.
+constexpr int kResidentMinSteps = 16;
+
+// Kernel arguments of nsteps steps of the bound shot from t0.
+Resident2D resident_args(const seis_model *m, int t0, int nsteps) {
+    Resident2D T;
+    std::memset(&T, 0, sizeof(T));
+    const FDArgs<float> &a = m->a;
+    T.g = m->g;
+    for (int k = 0; k < 7; ++k) T.hc[k] = a.hc[k];
+    T.DT = a.DT;
+    T.DT2 = a.DT2;
+    T.L = a.L;
+    for (int l = 0; l < std::min(a.L, 2); ++l) {
+        T.eta[l] = a.eta[l];
+        T.bl[l] = a.bl[l];
+        T.cl[l] = a.cl[l];
+    }
+    T.abs_type = a.abs_type;
+    T.freesurf = a.freesurf;
+    T.nab = a.nab;
+    if (m->nd_case == 22) {
+        float *f[] = {a.vx, a.vz, a.p}, *p[] = {a.psi_p_z, a.psi_p_x, a.psi_vz_z, a.psi_vx_x};
+        const float *c[] = {a.rip, a.rkp, a.M};
+        std::copy(f, f + 3, T.f);
+        std::copy(p, p + 4, T.p);
+        std::copy(c, c + 3, T.co);
+    } else {
+        float *f[] = {a.vx, a.vz, a.sxx, a.szz, a.sxz}, *r[] = {a.rxx, a.rzz, a.rxz};
+        float *p[] = {a.psi_sxz_z, a.psi_szz_z, a.psi_sxx_x, a.psi_sxz_x,
+                      a.psi_vx_z,  a.psi_vz_z,  a.psi_vx_x,  a.psi_vz_x};
+        const float *ce[] = {a.rip, a.rkp, a.M, a.mu, a.muipkp};
+        const float *cv[] = {a.rip, a.rkp, a.cg, a.cf, a.cd, a.ce, a.fipkp, a.dipkp};
+        std::copy(f, f + 5, T.f);
+        std::copy(r, r + 3, T.m);
+        std::copy(p, p + 8, T.p);
+        if (a.L) std::copy(cv, cv + 8, T.co);
+        else std::copy(ce, ce + 5, T.co);
+    }
+    T.cpml = a.cpml;
+    T.taper = a.taper;
+    T.s = m->shot;
+    T.NT = m->c.NT;
+    T.nout = (int)m->out_codes.size();
+    for (int q = 0; q < T.nout && q < 10; ++q) {
+        T.code[q] = m->out_codes[q];
+        T.unscale[q] = m->unscale.empty() ? 1.0f : m->unscale[q];
+    }
+    T.t0 = t0;
+    T.nsteps = nsteps;
+    return T;
+}
+
+// Whether a run of nsteps steps of the bound shot can stay on the chip: 2D,
+// wavefields in 32 bits, up to two Maxwell bodies, source and receiver tables
+// that fit a block's lists, a grid that fits the CUs.
+bool resident_covers(const seis_model *m, int nsteps) {
+    if (m->nd_case == 3 || (m->prec != P_FP32 && m->prec != P_SCALED) || !m->ctx->resident.ncu ||
+        m->c.L > (m->nd_case == 22 ? 0 : 2) || nsteps < kResidentMinSteps ||
+        m->shot.nsrc > kResidentMaxSrc || m->shot.nrec > kResidentMaxRec)
+        return false;
+    Resident2D T = resident_args(m, 0, nsteps);
+    return launch_resident2d(T, m->nd_case, m->ctx->resident.ncu, nullptr, nullptr);
+}
+
+// Makes the run T describes on the compute stream and waits for it.  *done: 1
+// if it was made, 0 if it gave up (the model's state is as before and the
+// caller makes the steps with the step kernels).  ms: device time, if wanted.
+int resident_run(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
+    seis_ctx *ctx = m->ctx;
+    seis_ctx::Resident &R = ctx->resident;
+    hipStream_t st = ctx->stream;
+    std::lock_guard<std::mutex> lock(R.mu);
+    // words, then the two counters
+    const size_t words = (m->nd_case == 22 ? 2 : kResidentWords) * (size_t)m->g.nfield * 8;
+    const size_t need = words + 64;
+    if (!R.failed) {
+        void *p = nullptr;
+        HIP_TRY(hipHostMalloc(&p, 64, hipHostMallocMapped));
+        R.failed = (int *)p;
+    }
+    if (need > R.bytes) {
+        if (R.words) ctx->release(R.words);
+        R.words = nullptr;
+        R.bytes = 0;
+        if (ctx->alloc(need, &R.words)) return 1;
+        R.bytes = need;
+    }
+    launch_fill(R.words, need, st);
+    *R.failed = 0;
+    void *fd = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&fd, R.failed, 0));
+    T.xch = (unsigned long long *)R.words;
+    T.sync = (int *)((char *)R.words + words);
+    T.patience = R.patience;
+    T.failed = (int *)fd;
+    hipEvent_t e0 = pool_event(m, 0), e1 = pool_event(m, 1);
+    if (!e0 || !e1) return fail("hipEventCreate failed");
+    HIP_TRY(hipEventRecord(e0, st));
+    int e = 0;
+    const bool fits = launch_resident2d(T, m->nd_case, R.ncu, st, &e);
+    if (!fits || e != hipSuccess) {
+        (void)hipGetLastError();
+        R.ncu = 0;
+        *done = 0;
+        return 0;
+    }
+    HIP_TRY(hipEventRecord(e1, st));
+    HIP_TRY(hipEventSynchronize(e1));
+    *done = !*(volatile int *)R.failed;
+    if (!*done) R.ncu = 0;
+    if (ms) HIP_TRY(hipEventElapsedTime(ms, e0, e1));
+    return 0;
+}
+
+// Steps t0 .. t0 + n - 1 of a gradient's forward run as one resident run, if it
+// covers them: with receivers (rec), the boundary shell of every step (bnd) or
+// the state after every step's sources (hist).  *done as resident_run.
+int resident_steps(seis_model *m, int t0, int n, bool rec, float *bnd, const Shell *sh,
+                   float *hist, int *done) {
+    *done = 0;
+    if (m->profiling || !resident_covers(m, n)) return 0;
+    Resident2D T = resident_args(m, t0, n);
+    if (!rec) T.s.nrec = 0;
+    T.bnd = bnd;
+    if (sh) T.sh = *sh;
+    T.hist = hist;
+    return resident_run(m, T, done);
+}
+
 // What a captured step sequence depends on: the kernel arguments (model
 // arguments, shot tables, outputs and their scales) and the precision.
 uint64_t step_key(const seis_model *m) {
@@ -948,6 +1093,20 @@ int seis_ctx_create(int device_ordinal, seis_ctx **out) {
     if (scratch_address(device_ordinal, &ctx->scratch)) return 1;
     HIP_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&ctx->xfer, hipStreamNonBlocking));
+    // SEIS_RESIDENT_WAIT_MS: longest wait of a block of a resident run for
+    // another block (default 500); a run that waits longer is made again by the
+    // step kernels, as are all later ones of the context
+    int coop = 0, ncu = 0, khz = 0;
+    const char *wait = getenv("SEIS_RESIDENT_WAIT_MS");
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_ordinal) != hipSuccess ||
+        khz <= 0)
+        khz = 100000;
+    ctx->resident.patience = (long long)(wait && *wait ? std::max(0, atoi(wait)) : 500) * khz;
+    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device_ordinal) ==
+            hipSuccess && coop &&
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device_ordinal) ==
+            hipSuccess)
+        ctx->resident.ncu = ncu;
     *out = ctx.release();
     return 0;
 }
@@ -958,6 +1117,7 @@ int seis_ctx_destroy(seis_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->xfer);
     for (auto &kv : ctx->caps) (void)hipFree(kv.first);
+    if (ctx->resident.failed) (void)hipHostFree(ctx->resident.failed);
     for (auto &kv : ctx->cache) (void)hipEventDestroy(kv.second.second);
     (void)hipStreamDestroy(ctx->stream);
     (void)hipStreamDestroy(ctx->xfer);
@@ -1364,6 +1524,17 @@ int seis_run_steps(seis_model *m, int t0, int nsteps) {
     if (!e0 || !e1) return fail("hipEventCreate failed");
     const bool prof = m->profiling;
     if (prof && !pool_event(m, 2 + 4 * (size_t)nsteps)) return fail("hipEventCreate failed");
+    if (!prof && resident_covers(m, nsteps)) {
+        Resident2D T = resident_args(m, t0, nsteps);
+        int done = 0;
+        float ms = 0;
+        if (resident_run(m, T, &done, &ms)) return 1;
+        if (done) {
+            m->ms_loop = ms;
+            m->ms_v = m->ms_s = 0;
+            return 0;
+        }
+    }
     // 2D runs without per-kernel events replay captured step graphs
     const bool graph = !prof && m->c.ND != 3 && nsteps >= kGraphSteps && graph_enabled();
     if (graph && graph_prepare(m, st)) return 1;
@@ -1723,15 +1894,19 @@ static int forward_save_visco(seis_model *m, float *out) {
     const CkptPlan &P = G.plan;
     const auto state = forward_state(m);
     const size_t sbytes = state_bytes(state);
-    for (int t = 0; t < tmax; ++t) {
-        if (t % P.K[0] == 0 &&
-            state_save(state, (char *)G.ckpt + (size_t)(t / P.K[0]) * sbytes, st))
-            return 1;
-        step_sources(m, t, 1, st);
-        step_v(m, st);
-        step_s(m, st);
-        if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
-        step_varsout(m, t, st);
+    for (int t0 = 0; t0 < tmax; t0 += P.K[0]) {
+        const int n = std::min(P.K[0], tmax - t0);
+        if (state_save(state, (char *)G.ckpt + (size_t)(t0 / P.K[0]) * sbytes, st)) return 1;
+        int done = 0;
+        if (resident_steps(m, t0, n, true, nullptr, nullptr, nullptr, &done)) return 1;
+        if (done) continue;
+        for (int t = t0; t < t0 + n; ++t) {
+            step_sources(m, t, 1, st);
+            step_v(m, st);
+            step_s(m, st);
+            if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
+            step_varsout(m, t, st);
+        }
     }
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
@@ -1793,10 +1968,13 @@ struct ViscoAdj {
         if (l == P.L - 1) return innermost(t0, t1);
         const int K = P.K[l + 1], nsub = (t1 - t0 + K - 1) / K;
         char *slots = (char *)G.ckpt + ((size_t)P.n0 + (size_t)l * (P.n - 1)) * sbytes;
-        for (int t = t0; t < t0 + (nsub - 1) * K; ++t) {
-            if ((t - t0) % K == 0 && state_save(state, slots + (size_t)((t - t0) / K) * sbytes, st))
-                return 1;
-            step_forward(m, t, st);
+        for (int s = 0; s < nsub - 1; ++s) {
+            const int u0 = t0 + s * K;
+            if (state_save(state, slots + (size_t)s * sbytes, st)) return 1;
+            int done = 0;
+            if (resident_steps(m, u0, K, false, nullptr, nullptr, nullptr, &done)) return 1;
+            if (!done)
+                for (int t = u0; t < u0 + K; ++t) step_forward(m, t, st);
         }
         for (int s = nsub - 1; s >= 0; --s) {
             const int u0 = t0 + s * K, u1 = std::min(u0 + K, t1);
@@ -1814,7 +1992,9 @@ struct ViscoAdj {
         const seis_csts &c = m->c;
         hipStream_t st = m->ctx->stream;
         const int NT = c.NT, nout = (int)m->outn.size();
-        for (int t = t0; t < t1; ++t) {
+        int done = 0;
+        if (!mv && resident_steps(m, t0, t1 - t0, false, nullptr, nullptr, G.hist, &done)) return 1;
+        for (int t = t0; t < t1 && !done; ++t) {
             // movie frame: the recomputed forward state at the start of step
             // t, what backpropagation reconstructs after the adjoint step t
             if (t > tmin && movie_snap(m, mv, t)) return 1;
@@ -2214,9 +2394,11 @@ int seis_forward_save(seis_model *m, int nsrc, const float *src_pos, const float
                            (long)per);
         if (m->c.freesurf) step_surface(m, st);
     };
-    int t0 = 0;
+    int t0 = 0, done = 0;
+    if (resident_steps(m, 0, tmax, true, G.bnd, &G.sh, nullptr, &done)) return 1;
+    if (done) t0 = tmax;
     // 2D: runs of kGraphSteps steps replayed from a captured graph
-    if (m->c.ND != 3 && !m->profiling && tmax >= kGraphSteps && graph_enabled()) {
+    if (!done && m->c.ND != 3 && !m->profiling && tmax >= kGraphSteps && graph_enabled()) {
         if (step_counter(m)) return 1;
         uint64_t key = step_key(m);
         key = key_mix(key, &G.bnd, sizeof(G.bnd));
@@ -2232,7 +2414,7 @@ int seis_forward_save(seis_model *m, int nsrc, const float *src_pos, const float
             HIP_TRY(hipGraphLaunch(m->fs_graph.e, st));
     }
     for (int t = t0; t < tmax; ++t) step(t, nullptr);
-    step_io(m, tmax - 1, -1, st);   // varsout of the last step
+    if (!done) step_io(m, tmax - 1, -1, st);   // varsout of the last step
     m->a.fuse_surface = fused;
     m->ad.fuse_surface = fused;
     HIP_TRY(hipGetLastError());

@@ -377,6 +377,48 @@ struct AdjArgs {
     long bofs = 0, bper = 0;
 };
 
+// ---------------------------------------------------------------------------
+// 2D runs resident on the chip (fd2d_resident.hip): FP32, L <= 2 (acoustic
+// L = 0).
+// ---------------------------------------------------------------------------
+constexpr int kResidentMaxRec = 1024, kResidentMaxSrc = 64, kResidentWords = 4;
+struct Resident2D {
+    Layout g;
+    float hc[7];
+    float DT, DT2;
+    int L;
+    float eta[2], bl[2], cl[2];
+    int abs_type, freesurf, nab;
+    // the state: vx vz sxx szz sxz (acoustic: vx vz p), memory variables rxx
+    // rzz rxz (L slabs each), CPML memory of the velocities then of the
+    // stresses, z strips before x strips
+    float *f[5], *m[3], *p[8];
+    // rip rkp, then M mu muipkp or g f d e fipkp dipkp (acoustic: rip rkp M)
+    const float *co[8];
+    const float *cpml, *taper;
+    ShotDev s;
+    int NT, nout, code[10];
+    float unscale[10];
+    int t0, nsteps;
+    // boundary shell of every step (bnd + t * 5 * sh.n) or null; state after
+    // the sources of step t0 + k at hist + k * 5 fields or null
+    float *bnd;
+    Shell sh;
+    float *hist;
+    // exchange words (kResidentWords per cell), zero; sync[2], zero: blocks
+    // done, the run's state; failed (host memory): set to 1 by a run that gave
+    // up
+    unsigned long long *xch;
+    int *sync, *failed;
+    long long patience;         // wall_clock64 ticks a block waits for another
+    // set by the launcher
+    int cz, cx, nbz;
+    unsigned ntile;
+};
+// Steps t0 .. t0 + nsteps - 1 on ncu CUs; false: the grid does not fit.  err:
+// the launch's hipError_t.  stream null: nothing is launched.
+bool launch_resident2d(Resident2D &a, int nd_case, int ncu, void *stream, int *err);
+
 // DFT-domain gradient (dft.hip).  The arrays whose spectra are kept:
 // velocities, stresses, then each memory-variable component's L slabs.
 struct DftArrays {
