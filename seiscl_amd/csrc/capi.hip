@@ -44,6 +44,8 @@ static __device__ __align__(256) unsigned char scratch[SEIS_STATIC_SHOT_BYTES];
 namespace {
 constexpr int kMaxDevices = 64;
 void *g_scratch_dev[kMaxDevices] = {};
+// one resident run at a time on a GPU: two would wait for each other's CUs
+std::mutex g_resident_mu[kMaxDevices];
 std::mutex g_scratch_mu;
 
 // Device address of this GPU's static area (the device must be current).
@@ -102,14 +104,15 @@ struct seis_ctx {
         hipEvent_t freed;           // compute-stream point after the last use
     };
     // workspace of resident 2D runs (fd2d_resident.hip): exchange words and the
-    // run's counters, a host word that a run which gave up sets.  One run at a time uses it (mu).
+    // run's counters, a host word that a run which gave up sets.  Used under
+    // the GPU's g_resident_mu.
     struct Resident {
         std::mutex mu;
         void *words = nullptr;
         size_t bytes = 0;
         int *failed = nullptr;      // pinned host memory
-        // CUs; 0: no resident runs (no cooperative launch, or a run gave up:
-        // the GPU is shared with another program's kernels)
+        // CUs; 0: no resident runs (a run gave up: the GPU is shared with another
+        // program's kernels)
         int ncu = 0;
         // longest wait of a block for another, in wall_clock64 ticks
         long long patience = 0;
@@ -708,17 +711,20 @@ bool resident_covers(const seis_model *m, int nsteps) {
     return launch_resident2d(T, m->nd_case, m->ctx->resident.ncu, nullptr, nullptr);
 }
 
-// Makes the run T describes on the compute stream and waits for it.  *done: 1
-// if it was made, 0 if it gave up (the model's state is as before and the
-// caller makes the steps with the step kernels).  ms: device time, if wanted.
-int resident_run(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
+// Makes a resident run on the compute stream and waits for it: launch(T, err)
+// launches it with T's workspace pointers set.  nw: exchange words per cell.
+// *done: 1 if the run was made, 0 if it gave up (the model's state is as before
+// and the caller makes the steps with the step kernels).  ms: device time, if
+// wanted.
+template <typename Args, typename F>
+int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launch) {
     seis_ctx *ctx = m->ctx;
     seis_ctx::Resident &R = ctx->resident;
     hipStream_t st = ctx->stream;
-    std::lock_guard<std::mutex> lock(R.mu);
+    std::lock_guard<std::mutex> lock(g_resident_mu[ctx->device]);
+    *done = 0;
     // words, then the two counters
-    const size_t words = (m->nd_case == 22 ? 2 : kResidentWords) * (size_t)m->g.nfield * 8;
-    const size_t need = words + 64;
+    const size_t words = (size_t)nw * m->g.nfield * 8, need = words + 64;
     if (!R.failed) {
         void *p = nullptr;
         HIP_TRY(hipHostMalloc(&p, 64, hipHostMallocMapped));
@@ -739,15 +745,14 @@ int resident_run(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
     T.sync = (int *)((char *)R.words + words);
     T.patience = R.patience;
     T.failed = (int *)fd;
-    hipEvent_t e0 = pool_event(m, 0), e1 = pool_event(m, 1);
+    // (events 0 and 1 time the caller's loop)
+    hipEvent_t e0 = pool_event(m, 2), e1 = pool_event(m, 3);
     if (!e0 || !e1) return fail("hipEventCreate failed");
     HIP_TRY(hipEventRecord(e0, st));
     int e = 0;
-    const bool fits = launch_resident2d(T, m->nd_case, R.ncu, st, &e);
-    if (!fits || e != hipSuccess) {
+    if (!launch(T, &e) || e != hipSuccess) {
         (void)hipGetLastError();
         R.ncu = 0;
-        *done = 0;
         return 0;
     }
     HIP_TRY(hipEventRecord(e1, st));
@@ -756,6 +761,11 @@ int resident_run(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
     if (!*done) R.ncu = 0;
     if (ms) HIP_TRY(hipEventElapsedTime(ms, e0, e1));
     return 0;
+}
+int resident_forward(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
+    return resident_run(m, T, m->nd_case == 22 ? 2 : 4, done, ms, [&](Resident2D &A, int *e) {
+        return launch_resident2d(A, m->nd_case, m->ctx->resident.ncu, m->ctx->stream, e);
+    });
 }
 
 // Steps t0 .. t0 + n - 1 of a gradient's forward run as one resident run, if it
@@ -770,7 +780,7 @@ int resident_steps(seis_model *m, int t0, int n, bool rec, float *bnd, const She
     T.bnd = bnd;
     if (sh) T.sh = *sh;
     T.hist = hist;
-    return resident_run(m, T, done);
+    return resident_forward(m, T, done);
 }
 
 // What a captured step sequence depends on: the kernel arguments (model
@@ -1096,14 +1106,13 @@ int seis_ctx_create(int device_ordinal, seis_ctx **out) {
     // SEIS_RESIDENT_WAIT_MS: longest wait of a block of a resident run for
     // another block (default 500); a run that waits longer is made again by the
     // step kernels, as are all later ones of the context
-    int coop = 0, ncu = 0, khz = 0;
+    int ncu = 0, khz = 0;
     const char *wait = getenv("SEIS_RESIDENT_WAIT_MS");
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_ordinal) != hipSuccess ||
         khz <= 0)
         khz = 100000;
     ctx->resident.patience = (long long)(wait && *wait ? std::max(0, atoi(wait)) : 500) * khz;
-    if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device_ordinal) ==
-            hipSuccess && coop &&
+    if (device_ordinal < kMaxDevices &&
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device_ordinal) ==
             hipSuccess)
         ctx->resident.ncu = ncu;
@@ -1528,7 +1537,7 @@ int seis_run_steps(seis_model *m, int t0, int nsteps) {
         Resident2D T = resident_args(m, t0, nsteps);
         int done = 0;
         float ms = 0;
-        if (resident_run(m, T, &done, &ms)) return 1;
+        if (resident_forward(m, T, &done, &ms)) return 1;
         if (done) {
             m->ms_loop = ms;
             m->ms_v = m->ms_s = 0;
@@ -1948,6 +1957,92 @@ static int movie_snap(seis_model *m, const MovieOut *mv, int t) {
 // Viscoelastic adjoint over the plan of forward_save_visco (R: float, or
 // double in FP64 runs).
 extern "C++" {
+// The adjoint steps t1, t1 - 1, ... t1 - n + 1 as one resident run, if it covers
+// them: 2D, adjoint fields in 32 bits, at most two Maxwell bodies, no Cerjan
+// taper, no RTM image, Hessian or per-node terms, receivers on cells of their
+// own.  hist (L > 0): the states of the steps from hist_t0 on.  *done as
+// resident_run; *surface: the first step's adjoint free surface has been
+// applied, whether the run was made or gave up.
+template <typename R>
+static int resident_adjoint(seis_model *m, const AdjArgs<R> &A, int t1, int n, int serial,
+                            const float *hist, int hist_t0, int *done, bool *surface) {
+    *done = 0;
+    *surface = false;
+    if constexpr (sizeof(R) == 4) {
+        auto &G = m->grad;
+        const seis_csts &c = m->c;
+        const int ncu = m->ctx->resident.ncu, nout = (int)m->out_codes.size();
+        if (c.ND != 2 || m->prec == P_FP16 || m->profiling || !ncu || c.L > 2 ||
+            c.abs_type == 2 || A.rtm || A.hM || A.grz || serial || nout > 6 ||
+            n < kResidentMinSteps || m->shot.nsrc > kResidentMaxSrc ||
+            m->shot.nrec > kResidentMaxRec)
+            return 0;
+        ResidentAdj2D T;
+        std::memset(&T, 0, sizeof(T));
+        const FDArgs<float> &r = A.r, &f = A.f;
+        T.g = m->g;
+        for (int k = 0; k < 7; ++k) T.hc[k] = r.hc[k];
+        T.DT = r.DT;
+        T.DT2 = r.DT2;
+        for (int l = 0; l < c.L; ++l) {
+            T.eta[l] = r.eta[l];
+            T.bl[l] = r.bl[l];
+            T.cl[l] = r.cl[l];
+        }
+        T.abs_type = r.abs_type;
+        T.freesurf = r.freesurf;
+        T.nab = r.nab;
+        float *af[] = {r.vx, r.vz, r.sxx, r.szz, r.sxz}, *mv[] = {r.rxx, r.rzz, r.rxz};
+        float *ff[] = {f.vx, f.vz, f.sxx, f.szz, f.sxz};
+        float *ps[] = {r.psi_sxz_z, r.psi_szz_z, r.psi_sxx_x, r.psi_sxz_x,
+                       r.psi_vx_z,  r.psi_vz_z,  r.psi_vx_x,  r.psi_vz_x};
+        const float *ce[] = {r.rip, r.rkp, r.M, r.mu, r.muipkp};
+        const float *cv[] = {r.rip, r.rkp, r.cg, r.cf, r.cd, r.ce, r.fipkp, r.dipkp};
+        std::copy(af, af + 5, T.f);
+        std::copy(mv, mv + 3, T.m);
+        std::copy(ff, ff + 5, T.fw);
+        std::copy(ps, ps + 8, T.p);
+        if (c.L) std::copy(cv, cv + 8, T.co);
+        else std::copy(ce, ce + 5, T.co);
+        T.surfM = r.M;
+        T.surfmu = r.mu;
+        T.Ms = A.Ms;
+        T.mus = A.mus;
+        T.cpml = r.cpml;
+        T.s = m->shot;
+        T.res = G.res;
+        T.NT = c.NT;
+        T.nout = nout;
+        std::copy(m->out_codes.begin(), m->out_codes.end(), T.code);
+        T.t1 = t1;
+        T.nsteps = n;
+        T.bnd = G.bnd;
+        T.sh = G.sh;
+        T.hist = hist;
+        T.hist_t0 = hist_t0;
+        T.gM = A.gM;
+        T.gmu = A.gmu;
+        T.grho = A.grho;
+        T.gtp = A.gtp;
+        T.gts = A.gts;
+        T.gscale_s = A.gscale_s;
+        T.gscale_v = A.gscale_v;
+        T.s0 = A.s0;
+        if ((c.L && (!T.gtp || !T.gts || !hist)) ||
+            !launch_resident_adj2d(T, c.L, ncu, nullptr, nullptr))
+            return 0;
+        hipStream_t st = m->ctx->stream;
+        if (c.freesurf) {
+            launch_surface_adj(A.r, (R *)G.stmp, m->nd_case, c.gradfix & FIX_SURF_SYY, st);
+            *surface = true;
+        }
+        return resident_run(m, T, c.L ? 4 : 6, done, nullptr, [&](ResidentAdj2D &B, int *e) {
+            return launch_resident_adj2d(B, c.L, ncu, st, e);
+        });
+    }
+    return 0;
+}
+
 template <typename R>
 struct ViscoAdj {
     seis_model *m;
@@ -2006,8 +2101,14 @@ struct ViscoAdj {
             step_s(m, st);
             if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
         }
-        for (int t = t1 - 1; t >= std::max(t0, tmin + 1); --t) {
-            if (c.freesurf)
+        const int tl = std::max(t0, tmin + 1);
+        bool surface = false;
+        done = 0;
+        if (!mv && !prof && resident_adjoint(m, *A, t1 - 1, t1 - tl, serial, G.hist, t0, &done, &surface))
+            return 1;
+        if (done) k += (size_t)(t1 - tl);
+        for (int t = t1 - 1; t >= tl && !done; --t) {
+            if (c.freesurf && !(surface && t == t1 - 1))
                 launch_surface_adj(A->r, (R *)G.stmp, m->nd_case, c.gradfix & FIX_SURF_SYY, st);
             launch_residuals(A->r, m->nd_case, m->shot, m->out_codes.data(), nout, G.res, NT, t,
                              serial, st);
@@ -2577,8 +2678,9 @@ static int adjoint_loops(seis_model *m, const MovieOut *mv) {
     const R *bnd0 = (const R *)G.bnd;
     // adjoint step t (relative to *tb when tb is given; the shell of step
     // t-1), src/time_stepping.c:869-940
+    bool surface = false;   // applied for the first step already
     auto step = [&](int t, const int *tb) {
-        if (m->c.freesurf)
+        if (m->c.freesurf && !(surface && !tb && t == tmax - 1))
             launch_surface_adj(A.r, (R *)G.stmp, m->nd_case, m->c.gradfix & FIX_SURF_SYY, st);
         launch_residuals(A.r, m->nd_case, m->shot, m->out_codes.data(), nout, G.res, NT, t, serial,
                          st, tb);
@@ -2590,10 +2692,21 @@ static int adjoint_loops(seis_model *m, const MovieOut *mv) {
         launch_adj_v(A, m->nd_case, st);
         step_sources(m, t, -1, st, tb);
     };
-    int t = tmax - 1;
+    int t = tmax - 1, done = 0;
+    if (!mv && !prof &&
+        resident_adjoint(m, A, t, tmax - 1 - tmin, serial, nullptr, 0, &done, &surface))
+        return 1;
+    if (done) {
+        k = nst;
+        t = tmin;
+    } else if (surface) {
+        step(t, nullptr);   // without the surface, which the run has applied
+        --t;
+        ++k;
+    }
     // 2D without profiling or movie: runs of kGraphSteps adjoint steps
     // replayed from a captured graph, the counter holding the run's first t
-    if (m->c.ND != 3 && !prof && !mv && tmax - 1 - tmin >= kGraphSteps && graph_enabled()) {
+    if (!done && m->c.ND != 3 && !prof && !mv && t - tmin >= kGraphSteps && graph_enabled()) {
         if (step_counter(m)) return 1;
         AdjArgs<R> K = A;
         K.bnd = bnd0;

@@ -30,13 +30,17 @@
 // Halo cells of the grid do not change and are not exchanged, the image rows
 // apart.
 //
-// Every block must be on the chip at once: the launch is cooperative, with at
-// most one block per CU.  A block that waits longer than a.patience gives up,
-// so the grid ends in any case.  Results are written only once every block has
-// made its last step: the last one to get there sets the run's state to
-// "complete", a block that gives up sets it to "failed", whichever comes
-// first, and every block obeys it.  A failed run leaves the model's state as it
-// was, and the caller makes the steps with the ordinary kernels.
+// Every block must be on the chip at once: there is at most one per CU, and the
+// host makes one such run at a time on a GPU.  Kernels of other streams end and
+// make room.  Where another program holds CUs for good, a block that waits
+// longer than a.patience (wall_clock64 ticks) gives up, so the grid ends in any
+// case.  Results are written only once every block has made its last step: the
+// last one to get there sets the run's state to "complete", a block that gives
+// up sets it to "failed", whichever comes first, and every block obeys it.  A
+// failed run leaves the model's state as it was, and the caller makes the steps
+// with the ordinary kernels.  (A cooperative launch goes through a queue of its
+// own: with a second context in use, changing between it and the context's
+// stream took 1.3 ms per run.)
 //
 // One wave holds 64 consecutive z of N consecutive x of the core and its rim:
 // LDS rows are read without bank conflicts, the x-derivatives of a lane's N
@@ -62,105 +66,13 @@
 // Arithmetic: the cell updates of fd_kernels.hip, term by term.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <type_traits>
-
-#include "fd_common.hpp"
-#include "seis_internal.hpp"
+#include "resident2d.hpp"
 
 namespace seis {
 namespace {
 
-// x-derivatives of N consecutive cells; f: the lane's first cell in LDS.
-// PLUS: forward (Dp), else backward (Dm), with their terms and order.
-template <int H, int N, bool PLUS, int RZ>
-__device__ __forceinline__ void dx(const float *f, const float *hc, float *d) {
-    constexpr int W = N + 2 * H - 1, O = PLUS ? H - 1 : H;
-    float w[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) w[k] = f[(k - O) * RZ];
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        float acc = PLUS ? hc[1] * (w[j + O + 1] - w[j + O]) : hc[1] * (w[j + O] - w[j + O - 1]);
-#pragma unroll
-        for (int k = 2; k <= H; ++k)
-            acc = acc + (PLUS ? hc[k] * (w[j + O + k] - w[j + O - k + 1])
-                              : hc[k] * (w[j + O + k - 1] - w[j + O - k]));
-        d[j] = acc;
-    }
-}
-template <int H, bool PLUS>
-__device__ __forceinline__ float dz(const float *f, const float *hc) {
-    float acc = PLUS ? hc[1] * (f[1] - f[0]) : hc[1] * (f[0] - f[-1]);
-#pragma unroll
-    for (int k = 2; k <= H; ++k)
-        acc = acc + (PLUS ? hc[k] * (f[k] - f[1 - k]) : hc[k] * (f[k - 1] - f[-k]));
-    return acc;
-}
-
-struct Prof {       // CPML profile at one cell: K, a, b on the full and half grid
-    float K, a, b, Kh, ah, bh;
-};
-__device__ __forceinline__ Prof prof_load(const float *c, int n, int kf, int kh) {
-    return {c[CK * n + kf], c[CA * n + kf], c[CB * n + kf],
-            c[CKH * n + kh], c[CAH * n + kh], c[CBH * n + kh]};
-}
-// the same from the block's LDS copy, six values per profile index
-__device__ __forceinline__ Prof prof_x(const float *p, int kf, int kh) {
-    return {p[6 * kf + CK], p[6 * kf + CA], p[6 * kf + CB],
-            p[6 * kh + CKH], p[6 * kh + CAH], p[6 * kh + CBH]};
-}
-__device__ __forceinline__ void pmlf(float &d, float &psi, const Prof &p) {
-    psi = p.b * psi + p.a * d;
-    d = d / p.K + psi;
-}
-__device__ __forceinline__ void pmlh(float &d, float &psi, const Prof &p) {
-    psi = p.bh * psi + p.ah * d;
-    d = d / p.Kh + psi;
-}
-
-using Word = unsigned long long;
-__device__ __forceinline__ void put_word(Word *p, Word v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ Word get_word(const Word *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// the words of one cell: NE exchanged fields (1 or 3), step number tag > 0
-template <int NE>
-constexpr int nwords() { return NE == 1 ? 1 : 2; }
-template <int NE>
-__device__ __forceinline__ void put_cell(Word *X, long plane, long i, const float *v, unsigned tag) {
-    if constexpr (NE == 1) {
-        put_word(X + i, (Word)tag << 32 | __float_as_uint(v[0]));
-    } else {
-        const unsigned m = __float_as_uint(v[1]), t = tag << 16;
-        put_word(X + i, (Word)(t | m >> 16) << 32 | __float_as_uint(v[0]));
-        put_word(X + plane + i, (Word)(t | (m & 0xffff)) << 32 | __float_as_uint(v[2]));
-    }
-}
-template <int NE>
-__device__ __forceinline__ void get_cell(const Word *X, long plane, long i, Word *w) {
-#pragma unroll
-    for (int q = 0; q < nwords<NE>(); ++q) w[q] = get_word(X + q * plane + i);
-}
-template <int NE>
-__device__ __forceinline__ bool cell_ready(const Word *w, unsigned tag) {
-    if constexpr (NE == 1) return (unsigned)(w[0] >> 32) == tag;
-    else return (unsigned)(w[0] >> 48) == (tag & 0xffff) && (unsigned)(w[1] >> 48) == (tag & 0xffff);
-}
-template <int NE>
-__device__ __forceinline__ void cell_values(const Word *w, float *v) {
-    v[0] = __uint_as_float((unsigned)w[0]);
-    if constexpr (NE == 3) {
-        v[1] = __uint_as_float((unsigned)(w[0] >> 32) << 16 | ((unsigned)(w[1] >> 32) & 0xffff));
-        v[2] = __uint_as_float((unsigned)w[1]);
-    }
-}
-
-// cells of the rim that a block takes from others: z sides, x sides, corners
-constexpr int rim_cells(int H, int CX, int CZ) { return 4 * H * CX + 4 * H * CZ + 4 * H * H; }
-
+// ACOUSTIC: fields vx, vz, p (else vx, vz, sxx, szz, sxz); L Maxwell bodies
+// (elastic case only).  NW waves, N columns of x per lane.
 template <int H, bool ACOUSTIC, int L, int NW, int N>
 __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     // the region: 64 + 2H rows of z, NW N + 2H columns
@@ -308,36 +220,11 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
         if (lx < 2 * H || lx >= 2 * H + CX || lz < 2 * H || lz >= 2 * H + CZ) continue;
         rlist[atomicAdd(&rcount, 1)] = r << 13 | (lx * RZ + lz);
     }
-    // the rim cells this thread takes: LDS cell and place in the grid (-1: none)
+    // the rim cells this thread takes
     int rl[MR], ri[MR];
-    {
-        const int nz = 4 * H * CX, nx = 4 * H * CZ;
 #pragma unroll
-        for (int e = 0; e < MR; ++e) {
-            int q = tid + e * 64 * NW, lx = 0, lz = 0;
-            bool in = true;
-            if (q < nz) {
-                lz = q % (4 * H);
-                lx = 2 * H + q / (4 * H);
-                if (lz >= 2 * H) lz += CZ;
-            } else if ((q -= nz) < nx) {
-                lz = 2 * H + q % CZ;
-                lx = q / CZ;
-                if (lx >= 2 * H) lx += CX;
-            } else if ((q -= nx) < 4 * H * H) {
-                lz = H + q % (2 * H);
-                lx = H + q / (2 * H);
-                if (lz >= 2 * H) lz += CZ;
-                if (lx >= 2 * H) lx += CX;
-            } else {
-                in = false;
-            }
-            const int zz = rz0 + lz, xx = rx0 + lx;
-            in = in && zz >= (a.freesurf ? -H : 0) && zz < NZ && xx >= 0 && xx < NX;
-            rl[e] = lx * RZ + lz;
-            ri[e] = in ? (int)g.idx(zz, 0, xx) : -1;
-        }
-    }
+    for (int e = 0; e < MR; ++e)
+        rim_cell<H, RZ>(g, a.freesurf, CZ, CX, rz0, rx0, tid + e * 64 * NW, rl[e], ri[e]);
     __syncthreads();
     const int nr = rcount;
     const float *hc = a.hc;
@@ -631,68 +518,17 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
             }
         }
         if (last) break;
-        // the rim: a thread's first cell is waited for alone, the others are
-        // loaded once that is there (they are then, as a rule, too): polling
-        // all of them in vain would keep the memory path busy
-        bool ok = true;
-        {
-            Word v[MR][nwords<NE>()];
-            const long long start = wall_clock64();
-            auto take = [&](auto first, auto end) {
-                constexpr int E0 = decltype(first)::value, E1 = decltype(end)::value;
-                while (true) {
-                    bool wait = false;
+        const bool ok = take_rim<NE, MR>(X, g.nfield, tag, a.patience, ri, [&](int e, const float *u) {
 #pragma unroll
-                    for (int e = E0; e < E1; ++e)
-                        if (ri[e] >= 0) get_cell<NE>(X, g.nfield, ri[e], v[e]);
-#pragma unroll
-                    for (int e = E0; e < E1; ++e)
-                        if (ri[e] >= 0 && !cell_ready<NE>(v[e], tag)) wait = true;
-                    if (!__any(wait)) break;
-                    if (wall_clock64() - start > a.patience) return false;
-                }
-                return true;
-            };
-            ok = take(std::integral_constant<int, 0>(), std::integral_constant<int, 1>());
-            if constexpr (MR > 1)
-                ok = ok && take(std::integral_constant<int, 1>(), std::integral_constant<int, MR>());
-            if (ok) {
-#pragma unroll
-                for (int e = 0; e < MR; ++e)
-                    if (ri[e] >= 0) {
-                        float u[NE];
-                        cell_values<NE>(v[e], u);
-#pragma unroll
-                        for (int q = 0; q < NE; ++q) lds[(2 + q) * FS + rl[e]] = u[q];
-                    }
-            }
-        }
+            for (int q = 0; q < NE; ++q) lds[(2 + q) * FS + rl[e]] = u[q];
+        });
         if (!ok && lane == 0) dead = 1;
         __syncthreads();
         if (dead) break;
     }
 
     // every block's last step is made, or the run has failed
-    if (tid == 0) {
-        int st = dead ? 2 : 0;
-        if (!dead) {
-            if (__hip_atomic_fetch_add(a.sync, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
-                (int)a.ntile)
-                st = 1;
-            const long long start = wall_clock64();
-            while (!st) {
-                st = __hip_atomic_load(a.sync + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                if (!st && wall_clock64() - start > a.patience) st = 2;
-            }
-        }
-        int open = 0;
-        if (!__hip_atomic_compare_exchange_strong(a.sync + 1, &open, st, __ATOMIC_ACQ_REL,
-                                                  __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT))
-            st = open;
-        verdict = st;
-        if (st == 2)
-            __hip_atomic_store(a.failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (tid == 0) verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience);
     __syncthreads();
     if (verdict != 1) return;
 
@@ -719,28 +555,6 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     }
 }
 
-// Tiles of a grid for one instantiation: nbz x nbx blocks of cores CZ x CX.
-struct Tiling {
-    int nbz = 0, nbx = 0, cz = 0, cx = 0;
-};
-// The fewest rows of tiles, evenly high, then as many columns as the chip has
-// CUs for, but no core narrower than kMinCX.
-constexpr int kMinCX = 4;
-Tiling tiling(const Layout &g, int cols, int ncu) {
-    Tiling t;
-    const int H = g.H, nz = g.NZ + 2 * H, nx = g.NX + 2 * H, czm = 64 - 2 * H, cxm = cols - 2 * H;
-    ncu = ncu / 8 * 8;   // the launch rounds the number of blocks up to 8
-    if (cxm < 1 || ncu < 8) return t;
-    t.nbz = (nz + czm - 1) / czm;
-    t.cz = std::max((nz + t.nbz - 1) / t.nbz, 2 * H + 1);
-    t.nbz = (nz + t.cz - 1) / t.cz;
-    if (t.nbz > ncu) return Tiling();
-    t.cx = std::max(kMinCX, (nx + ncu / t.nbz - 1) / (ncu / t.nbz));
-    if (t.cx > cxm) return Tiling();
-    t.nbx = (nx + t.cx - 1) / t.cx;
-    return t;
-}
-
 template <int H, bool ACOUSTIC, int L, int NW, int N>
 bool run_resident(Resident2D &a, int ncu, hipStream_t st, int &err) {
     const Tiling t = tiling(a.g, NW * N, ncu);
@@ -750,10 +564,8 @@ bool run_resident(Resident2D &a, int ncu, hipStream_t st, int &err) {
     a.nbz = t.nbz;
     a.ntile = (unsigned)(t.nbz * t.nbx);
     if (!st) return true;
-    void *args[] = {&a};
-    err = (int)hipLaunchCooperativeKernel(
-        reinterpret_cast<const void *>(&k_resident2d<H, ACOUSTIC, L, NW, N>),
-        dim3((a.ntile + 7) / 8 * 8), dim3(64, NW), args, 0, st);
+    hipLaunchKernelGGL((k_resident2d<H, ACOUSTIC, L, NW, N>), dim3((a.ntile + 7) / 8 * 8), dim3(64, NW), 0, st, a);
+    err = (int)hipGetLastError();
     return true;
 }
 
@@ -781,8 +593,7 @@ bool dispatch(Resident2D &a, int nd_case, int ncu, hipStream_t st, int &err) {
                 run_resident<H, false, 1, 16, 2>(a, ncu, st, err))
                 return true;
             if constexpr (H <= 3)
-                return run_resident<H, false, 1, 16, 3>(a, ncu, st, err) ||
-                       run_resident<H, false, 1, 8, 10>(a, ncu, st, err);
+                return run_resident<H, false, 1, 16, 3>(a, ncu, st, err);
             else
                 return run_resident<H, false, 1, 8, 6>(a, ncu, st, err);
         case 2:

@@ -381,7 +381,7 @@ struct AdjArgs {
 // 2D runs resident on the chip (fd2d_resident.hip): FP32, L <= 2 (acoustic
 // L = 0).
 // ---------------------------------------------------------------------------
-constexpr int kResidentMaxRec = 1024, kResidentMaxSrc = 64, kResidentWords = 4;
+constexpr int kResidentMaxRec = 1024, kResidentMaxSrc = 64, kResidentWords = 6;
 struct Resident2D {
     Layout g;
     float hc[7];
@@ -405,7 +405,7 @@ struct Resident2D {
     float *bnd;
     Shell sh;
     float *hist;
-    // exchange words (kResidentWords per cell), zero; sync[2], zero: blocks
+    // exchange words (at most kResidentWords per cell), zero; sync[2], zero: blocks
     // done, the run's state; failed (host memory): set to 1 by a run that gave
     // up
     unsigned long long *xch;
@@ -418,6 +418,40 @@ struct Resident2D {
 // Steps t0 .. t0 + nsteps - 1 on ncu CUs; false: the grid does not fit.  err:
 // the launch's hipError_t.  stream null: nothing is launched.
 bool launch_resident2d(Resident2D &a, int nd_case, int ncu, void *stream, int *err);
+
+// The adjoint steps t1, t1 - 1, ... of a 2D elastic (L = 0) or viscoelastic
+// (L <= 2) gradient (adj2d_resident.hip).
+struct ResidentAdj2D {
+    Layout g;
+    float hc[7];
+    float DT, DT2;
+    float eta[2], bl[2], cl[2];
+    int abs_type, freesurf, nab;     // abs_type 0 or 1
+    // adjoint state and coefficients as Resident2D's; the forward wavefields
+    // (L = 0: run backwards)
+    float *f[5], *m[3], *p[8], *fw[5];
+    const float *co[8];
+    const float *surfM, *surfmu;     // moduli of the adjoint free surface
+    const float *Ms, *mus;           // L > 0: moduli of the gradient formulas
+    const float *cpml;
+    ShotDev s;
+    const float *res;                // adjoint sources [nout][nrec][NT]
+    int NT, nout, code[10];
+    int t1, nsteps;
+    const float *bnd;                // L = 0: boundary shell (bnd + t * 5 * sh.n)
+    Shell sh;
+    const float *hist;               // L > 0: state of step t at hist + (t - hist_t0) * 5 fields
+    int hist_t0;
+    double *gM, *gmu, *grho, *gtp, *gts;
+    double gscale_s, gscale_v;
+    float s0;
+    unsigned long long *xch;
+    int *sync, *failed;
+    long long patience;
+    int cz, cx, nbz;
+    unsigned ntile;
+};
+bool launch_resident_adj2d(ResidentAdj2D &a, int L, int ncu, void *stream, int *err);
 
 // DFT-domain gradient (dft.hip).  The arrays whose spectra are kept:
 // velocities, stresses, then each memory-variable component's L slabs.

@@ -96,6 +96,51 @@ def test_resident_runs_continue(gpu_ctx, case):
         assert np.array_equal(a, b)
 
 
+# Adjoint runs hold ten wavefields (elastic) in LDS: tiles 16, 32 or 48 - 2H
+# columns wide; viscoelastic ones 16 or 32.
+GRADS = (
+    [dict(ND=2, FDORDER=o, N=n) for o, n in (
+        (2, (36, 37)), (4, (56, 60)), (4, (113, 131)), (8, (49, 97)), (12, (91, 67)),
+        (4, (120, 900)), (4, (120, 1700)), (6, (120, 2100)), (8, (120, 2100)))]
+    + [dict(ND=2, FDORDER=o, N=(113, 140), L=l, freesurf=f, seisout=so)
+       for o, so in ((4, 2), (6, 1), (10, 4)) for l in (0, 1, 2) for f in (0, 1)]
+    + [dict(ND=2, FDORDER=4, N=(113, 1100), L=2, freesurf=1)]
+    + [dict(ND=2, FDORDER=8, N=(107, 111), abs_type=0, L=l) for l in (0, 2)]
+)
+
+
+def _gradient(m, shot, seed=5):
+    rp = shot[2]
+    rng = np.random.default_rng(seed)
+    m.grad_zero()
+    out = m.forward_save(*shot)
+    size = max(np.abs(o).max() for o in out)
+    res = [(size * rng.standard_normal((NT, rp.shape[1]))).astype(np.float32) for _ in out]
+    m.adjoint(res)
+    return m.grad_read(), _state(m, 2) if m.csts.L == 0 else []
+
+
+@pytest.mark.parametrize("case", GRADS, ids=_ids)
+def test_resident_adjoint_equals_steps(gpu_ctx, case):
+    from seiscl_amd import Model
+    csts, params, (sp, s, rp) = _shot(case)
+    # receivers on cells of their own (the others stay with the step kernels)
+    cells = rp[[0, 2]].astype(int).T
+    rp = rp[:, np.unique(cells, axis=0, return_index=True)[1]]
+    m = Model(gpu_ctx, params, **csts)
+    if case.get("L"):
+        m.set_grad_memory((100 << 20) if case["N"][1] > 1000 else 0)
+    g, f = _gradient(m, (sp, s, rp))
+    m.set_profiling(True)
+    r, rf = _gradient(m, (sp, s, rp))
+    m.close()
+    for k in r:
+        assert np.abs(r[k]).max() > 0
+        assert np.array_equal(g[k], r[k]), k
+    for a, b in zip(f, rf):
+        assert np.array_equal(a, b)
+
+
 def test_run_that_gives_up_is_made_by_steps(gpu_ctx, monkeypatch):
     """Blocks that do not wait at all: the run ends, the model's state is as
     before it, and the step kernels make the steps."""
@@ -113,5 +158,24 @@ def test_run_that_gives_up_is_made_by_steps(gpu_ctx, monkeypatch):
         got, fields = m.forward(*shot), _state(m, 2)
         for a, b in zip(got + fields, ref + rfields):
             assert np.array_equal(a, b)
+    m.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("L", [0, 1])
+def test_adjoint_that_gives_up_is_made_by_steps(gpu_ctx, monkeypatch, L):
+    from seiscl_amd import Context, Model
+    csts, params, (sp, s, rp) = _shot(dict(ND=2, FDORDER=4, N=(113, 140), L=L, freesurf=1))
+    rp = rp[:, :100]
+    m = Model(gpu_ctx, params, **csts)
+    r, _ = _gradient(m, (sp, s, rp))
+    m.close()
+    monkeypatch.setenv("SEIS_RESIDENT_WAIT_MS", "0")
+    ctx = Context(0)
+    m = Model(ctx, params, **csts)
+    for _ in range(2):
+        g, _ = _gradient(m, (sp, s, rp))
+        for k in r:
+            assert np.array_equal(g[k], r[k]), k
     m.close()
     ctx.close()
