@@ -163,6 +163,8 @@ int seis_launch_varsout(seis_model *m, int nt);
 /* D2H of the bound shot's seismograms, [nout][nrec][NT] (reduce_seis,       */
 /* src/time_stepping.c:25-90).                                                */
 int seis_shot_read(seis_model *m, float *out);
+/* The same time-major, [nout][NT][nrec], the order the receivers record in.  */
+int seis_shot_read_nt(seis_model *m, float *out);
 /* The same into device memory of the model's GPU, [nout][nrec][NT] floats  */
 /* (reduce_seis, src/time_stepping.c:25-90, without leaving the GPU).         */
 int seis_shot_read_device(seis_model *m, float *dout);
@@ -298,9 +300,13 @@ int seis_grad_read(seis_model *m, float *grad);
 /* accumulated in double by the time-domain adjoint kernels from the whole */
 /* memory term of each step.                                                */
 int seis_grad_read_tau(seis_model *m, float *gtau);
+/* seis_grad_read (grad not NULL) and seis_grad_read_tau (gtau not NULL)    */
+/* with the cells in SeisCL.py's array order, [NZ][NY][NX] (SeisCL.py's      */
+/* transposes of what src/writehdf5.c writes).                               */
+int seis_grad_read_model(seis_model *m, float *grad, float *gtau);
 /* seis_grad_read and (dgtau not NULL) seis_grad_read_tau into device       */
 /* memory of the model's GPU (gradout of src/time_stepping.c:948-1003 for a  */
-/* caller whose tensors live there); the transform runs on the host.         */
+/* caller whose tensors live there).                                          */
 int seis_grad_read_device(seis_model *m, float *dgrad, float *dgtau);
 /* The approximate Hessian accumulated with the gradient when Hout=1,       */
 /* [3][Pi N] in the same order and transform (H<name> of the gradient file,  */

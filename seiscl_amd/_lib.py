@@ -87,6 +87,7 @@ SIGNATURES = [
     ("seis_launch_surface", _I, [_P]),
     ("seis_launch_varsout", _I, [_P, _I]),
     ("seis_shot_read", _I, [_P, _FP]),
+    ("seis_shot_read_nt", _I, [_P, _FP]),
     ("seis_shot_read_device", _I, [_P, _P]),
     ("seis_shot_read_f64", _I, [_P, ctypes.POINTER(ctypes.c_double)]),
     ("seis_hess_read", _I, [_P, _FP]),
@@ -112,6 +113,7 @@ SIGNATURES = [
     ("seis_grad_dft", _I, [_P, _I, _FP]),
     ("seis_grad_read", _I, [_P, _FP]),
     ("seis_grad_read_tau", _I, [_P, _FP]),
+    ("seis_grad_read_model", _I, [_P, _FP, _FP]),
     ("seis_grad_read_device", _I, [_P, _P, _P]),
     ("seis_gradient_shot", _I, [_P, _I, _FP, _FP, _I, _FP, _FP, _FP, _FP,
                                 ctypes.POINTER(ctypes.c_double)]),

@@ -252,6 +252,8 @@ struct seis_model {
         size_t ckpt_bytes = 0, hist_bytes = 0;
         size_t mem_limit = 0;       // budget of ckpt + hist; 0: 90% of free memory
         float *Ms = nullptr, *mus = nullptr;   // moduli of the gradient formulas
+        float *rho = nullptr;       // buoyancy of the cells, padded
+        bool moduli = false;        // Ms, mus (viscoelastic) and rho are the model's
     } grad;
     // DFT-domain gradient (seis_grad_dft): sampling of the spectra, the
     // factor table, forward and adjoint spectra, the cell parameters
@@ -920,6 +922,8 @@ int grad_setup(seis_model *m) {
             if (!(*mv[q] = m->dalloc(nf * c.L))) return 1;
         if (!(G.Ms = m->dalloc(nf)) || !(G.mus = m->dalloc(nf))) return 1;
     }
+    if (!(G.rho = m->dalloc(m->g.nfield))) return 1;
+    G.moduli = false;
     // own adjoint CPML memory: zeroed (FIX_ADJ_CPML), or, for viscoelastic
     // runs whose forward memory is overwritten by the recomputation, a copy
     // of the forward run's final memory (what the reference's kernels bind)
@@ -1281,6 +1285,7 @@ int seis_model_set_params(seis_model *m, const float *p0, const float *p1, const
     if (upload_params(m, rp)) return 1;
     if (m->prec == P_FP64) m->ad = as_double(m->a);
     m->rp = std::move(rp);
+    m->grad.moduli = false;
     return 0;
 }
 
@@ -1517,6 +1522,34 @@ static int shot_read(seis_model *m, float *outf, double *outd) {
 }  // namespace
 
 int seis_shot_read(seis_model *m, float *out) { return shot_read(m, out, nullptr); }
+
+int seis_shot_read_nt(seis_model *m, float *out) {
+    g_err.clear();
+    const int NT = m->c.NT, nrec = m->shot.nrec, nout = (int)m->outn.size();
+    const size_t n = (size_t)NT * nout * nrec;
+    if (!n) return 0;
+    if (!m->shot.out) return fail("seis_shot_read_nt: no shot bound");
+    hipStream_t st = m->ctx->stream;
+    if (m->done_ev) {   // as shot_read
+        st = m->ctx->xfer;
+        HIP_TRY(hipStreamWaitEvent(st, m->done_ev, 0));
+    }
+    const bool dbl = m->prec == P_FP64;
+    const float *src = m->shot.out;
+    void *p = nullptr;
+    if (nout > 1 || dbl) {
+        if (m->ctx->alloc(n * 4, &p, st)) return 1;
+        launch_seis_rows(m->shot.out, dbl, (float *)p, NT, nout, nrec, st);
+        src = (const float *)p;
+    }
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(out, src, n * 4, hipMemcpyDeviceToHost, st);
+    const hipError_t e2 = hipStreamSynchronize(st);
+    m->ctx->release(p);
+    if (e != hipSuccess || e2 != hipSuccess)
+        return fail(std::string("seis_shot_read_nt: ") + hipGetErrorString(e != hipSuccess ? e : e2));
+    return 0;
+}
 
 int seis_shot_read_f64(seis_model *m, double *out) {
     g_err.clear();
@@ -1816,20 +1849,30 @@ static size_t state_bytes(const std::vector<std::pair<float *, size_t>> &st) {
     for (auto &e : st) b += e.second;
     return b;
 }
-static int state_save(const std::vector<std::pair<float *, size_t>> &st, char *dst, hipStream_t s) {
+// One launch for all arrays of a state: a copy call each costs more than the copy
+// on grids of up to a few hundred thousand cells.
+static int state_copy(const std::vector<std::pair<float *, size_t>> &st, char *buf, bool save,
+                      hipStream_t s) {
+    CopyList c;
     for (auto &e : st) {
-        HIP_TRY(hipMemcpyAsync(dst, e.first, e.second, hipMemcpyDeviceToDevice, s));
-        dst += e.second;
+        if (c.n == kCopyMax) {
+            launch_copy_list(c, s);
+            c.n = 0;
+        }
+        c.src[c.n] = save ? (const void *)e.first : buf;
+        c.dst[c.n] = save ? (void *)buf : e.first;
+        c.bytes[c.n++] = e.second;
+        buf += e.second;
     }
+    launch_copy_list(c, s);
     return 0;
+}
+static int state_save(const std::vector<std::pair<float *, size_t>> &st, char *dst, hipStream_t s) {
+    return state_copy(st, dst, true, s);
 }
 static int state_load(const std::vector<std::pair<float *, size_t>> &st, const char *src,
                hipStream_t s) {
-    for (auto &e : st) {
-        HIP_TRY(hipMemcpyAsync(e.first, src, e.second, hipMemcpyDeviceToDevice, s));
-        src += e.second;
-    }
-    return 0;
+    return state_copy(st, const_cast<char *>(src), false, s);
 }
 
 // One forward step without receivers (the recomputations).
@@ -1840,30 +1883,44 @@ static void step_forward(seis_model *m, int t, hipStream_t st) {
     if (m->c.freesurf && !m->a.fuse_surface) step_surface(m, st);
 }
 
+// The moduli of the gradient formulas and the buoyancy on the device, once per
+// set of parameters.
+static int grad_moduli(seis_model *m) {
+    auto &G = m->grad;
+    if (G.moduli) return 0;
+    const seis_csts &c = m->c;
+    hipStream_t st = m->ctx->stream;
+    // moduli at f0 (FIX_VISCO_F0) or relaxed
+    const bool f0 = c.gradfix & FIX_VISCO_F0;
+    std::vector<float> h;
+    std::vector<double> hd;
+    if (G.visco)
+        for (int q = 0; q < 2; ++q) {
+            const std::vector<float> &v = f0 ? (q ? m->rp.muf0 : m->rp.Mf0) : (q ? m->rp.mu : m->rp.M);
+            to_padded(m->g, v.data(), 1.0f, h);
+            const void *src = h.data();
+            size_t bytes = h.size() * 4;
+            if (m->prec == P_FP64) {   // FP64 runs read the moduli in double
+                hd.assign(h.begin(), h.end());
+                src = hd.data();
+                bytes = hd.size() * 8;
+            }
+            HIP_TRY(hipMemcpyAsync(q ? G.mus : G.Ms, src, bytes, hipMemcpyHostToDevice, st));
+            HIP_TRY(hipStreamSynchronize(st));
+        }
+    to_padded(m->g, m->rp.rho.data(), 1.0f, h);
+    HIP_TRY(hipMemcpyAsync(G.rho, h.data(), h.size() * 4, hipMemcpyHostToDevice, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    G.moduli = true;
+    return 0;
+}
+
 // Set-up of a viscoelastic gradient run: the moduli of the gradient
 // formulas, the checkpoint plan and its buffers.
 static int visco_prepare(seis_model *m) {
     auto &G = m->grad;
-    const seis_csts &c = m->c;
     const int tmax = tmax_of(m);
-    hipStream_t st = m->ctx->stream;
-    // moduli of the gradient formulas: at f0 (FIX_VISCO_F0) or relaxed
-    const bool f0 = c.gradfix & FIX_VISCO_F0;
-    const std::vector<float> &Ms = f0 ? m->rp.Mf0 : m->rp.M, &mus = f0 ? m->rp.muf0 : m->rp.mu;
-    std::vector<float> h;
-    std::vector<double> hd;
-    for (int q = 0; q < 2; ++q) {
-        to_padded(m->g, (q ? mus : Ms).data(), 1.0f, h);
-        const void *src = h.data();
-        size_t bytes = h.size() * 4;
-        if (m->prec == P_FP64) {   // FP64 runs read the moduli in double
-            hd.assign(h.begin(), h.end());
-            src = hd.data();
-            bytes = hd.size() * 8;
-        }
-        HIP_TRY(hipMemcpyAsync(q ? G.mus : G.Ms, src, bytes, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipStreamSynchronize(st));
-    }
+    if (grad_moduli(m)) return 1;
     const auto state = forward_state(m);
     const size_t sbytes = state_bytes(state);
     const size_t hbytes = (size_t)G.nvb * m->g.nfield * m->selem;
@@ -2095,8 +2152,14 @@ struct ViscoAdj {
             if (t > tmin && movie_snap(m, mv, t)) return 1;
             step_sources(m, t, 1, st);
             char *dst = (char *)G.hist + (size_t)(t - t0) * G.nvb * fb;
-            for (size_t q = 0; q < hf.size(); ++q)
-                HIP_TRY(hipMemcpyAsync(dst + q * fb, hf[q], fb, hipMemcpyDeviceToDevice, st));
+            CopyList cl;
+            for (size_t q = 0; q < hf.size(); ++q) {
+                cl.src[q] = hf[q];
+                cl.dst[q] = dst + q * fb;
+                cl.bytes[q] = fb;
+            }
+            cl.n = (int)hf.size();
+            launch_copy_list(cl, st);
             step_v(m, st);
             step_s(m, st);
             if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
@@ -2916,8 +2979,10 @@ static int accum_read(seis_model *m, const double *const *src, int k, std::vecto
 }
 }  // namespace
 
-int seis_grad_read(seis_model *m, float *grad) {
-    g_err.clear();
+namespace {
+// seis_grad_read on the host: DFT gradients and gradients through the staggered
+// averages.
+static int grad_read_host(seis_model *m, float *grad) {
     auto &G = m->grad;
     if (!G.ready) return fail("seis_grad_read: no gradient accumulated");
     std::vector<double> acc[3];
@@ -2952,27 +3017,7 @@ int seis_grad_read(seis_model *m, float *grad) {
     return 0;
 }
 
-int seis_grad_read_device(seis_model *m, float *dgrad, float *dgtau) {
-    g_err.clear();
-    const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
-    hipStream_t st = m->ctx->stream;
-    if (dgrad) {
-        std::vector<float> h(3 * n);
-        if (seis_grad_read(m, h.data())) return 1;
-        HIP_TRY(hipMemcpyAsync(dgrad, h.data(), h.size() * 4, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipStreamSynchronize(st));
-    }
-    if (dgtau) {
-        std::vector<float> h(2 * n);
-        if (seis_grad_read_tau(m, h.data())) return 1;
-        HIP_TRY(hipMemcpyAsync(dgtau, h.data(), h.size() * 4, hipMemcpyHostToDevice, st));
-        HIP_TRY(hipStreamSynchronize(st));
-    }
-    return 0;
-}
-
-int seis_grad_read_tau(seis_model *m, float *gtau) {
-    g_err.clear();
+static int grad_read_tau_host(seis_model *m, float *gtau) {
     auto &G = m->grad;
     if (!G.ready || !G.gtp)
         return fail("seis_grad_read_tau: no tau gradient accumulated (viscoelastic runs, "
@@ -2995,6 +3040,132 @@ int seis_grad_read_tau(seis_model *m, float *gtau) {
     for (size_t i = 0; i < n; ++i) {
         gtau[i] = (float)(acc[0][i] * k);
         gtau[n + i] = (float)(acc[1][i] * k);
+    }
+    return 0;
+}
+
+
+bool grad_on_device(const seis_model *m) { return !m->dft.nf && !m->grad.grz; }
+
+int grad_check(const seis_model *m, bool tau) {
+    if (!m->grad.ready) return fail(tau ? "seis_grad_read_tau: no tau gradient accumulated (viscoelastic "
+                                          "runs, param_type 0-2)"
+                                        : "seis_grad_read: no gradient accumulated");
+    if (tau && !m->grad.gtp)
+        return fail("seis_grad_read_tau: no tau gradient accumulated (viscoelastic runs, "
+                    "param_type 0-2)");
+    return 0;
+}
+
+// Gradients (out [3][N], or null) and tau gradients (tau [2][N], or null) into
+// device memory, model: [NZ][NY][NX] instead of the parameter layout.
+int grad_device(seis_model *m, float *out, float *tau, int model) {
+    auto &G = m->grad;
+    if (grad_moduli(m)) return 1;
+    GradOut a;
+    std::memset(&a, 0, sizeof(a));
+    a.lay = m->g;
+    const double *g[5] = {G.gM, G.gmu, G.grho, G.gtp, G.gts};
+    std::copy(g, g + 5, a.g);
+    // elastic runs are never in scaled units: the update's moduli are the model's
+    a.Ms = G.visco ? (const void *)G.Ms : m->a.M;
+    a.mus = G.visco ? (const void *)G.mus : m->a.mu;
+    a.rho = G.rho;
+    a.dt = m->c.dt;
+    a.dh = m->c.dh;
+    // the accumulators hold dt^2/dh times dJ/dtau, as the moduli's hold
+    // dt^2/dh times the derivative by the scaled moduli (transf_grad)
+    a.ktau = (double)m->c.dh / ((double)m->c.dt * m->c.dt);
+    a.param_type = m->c.param_type;
+    a.rho_fix = (m->c.gradfix & FIX_RHO_SCALE) != 0;
+    a.model = model;
+    a.out = out;
+    a.tau = tau;
+    launch_grad_out(a, m->prec == P_FP64, m->ctx->stream);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// The same into host memory.
+int grad_to_host(seis_model *m, float *out, float *tau, int model) {
+    const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
+    hipStream_t st = m->ctx->stream;
+    void *p = nullptr;
+    if (m->ctx->alloc(((out ? 3 : 0) + (tau ? 2 : 0)) * n * 4, &p)) return 1;
+    float *dout = out ? (float *)p : nullptr, *dtau = tau ? (float *)p + (out ? 3 * n : 0) : nullptr;
+    int rc = grad_device(m, dout, dtau, model);
+    hipError_t e = hipSuccess;
+    if (!rc && out) e = hipMemcpyAsync(out, dout, 3 * n * 4, hipMemcpyDeviceToHost, st);
+    if (!rc && tau && e == hipSuccess)
+        e = hipMemcpyAsync(tau, dtau, 2 * n * 4, hipMemcpyDeviceToHost, st);
+    const hipError_t e2 = hipStreamSynchronize(st);
+    m->ctx->release(p);
+    if (rc) return rc;
+    if (e != hipSuccess || e2 != hipSuccess)
+        return fail(std::string("gradient read: ") + hipGetErrorString(e != hipSuccess ? e : e2));
+    return 0;
+}
+
+// [NX][NY][NZ] -> [NZ][NY][NX], k arrays
+void to_model_layout(const seis_model *m, const std::vector<float> &in, float *out, int k) {
+    const size_t NZ = m->g.NZ, NY = m->g.NY, NX = m->g.NX, n = NZ * NY * NX;
+    for (int q = 0; q < k; ++q)
+        for (size_t x = 0; x < NX; ++x)
+            for (size_t y = 0; y < NY; ++y)
+                for (size_t z = 0; z < NZ; ++z)
+                    out[q * n + (z * NY + y) * NX + x] = in[q * n + (x * NY + y) * NZ + z];
+}
+}  // namespace
+
+int seis_grad_read(seis_model *m, float *grad) {
+    g_err.clear();
+    if (grad_check(m, false)) return 1;
+    return grad_on_device(m) ? grad_to_host(m, grad, nullptr, 0) : grad_read_host(m, grad);
+}
+
+int seis_grad_read_tau(seis_model *m, float *gtau) {
+    g_err.clear();
+    if (grad_check(m, true)) return 1;
+    return grad_on_device(m) ? grad_to_host(m, nullptr, gtau, 0) : grad_read_tau_host(m, gtau);
+}
+
+int seis_grad_read_model(seis_model *m, float *grad, float *gtau) {
+    g_err.clear();
+    if (grad_check(m, false) || (gtau && grad_check(m, true))) return 1;
+    if (grad_on_device(m)) return grad_to_host(m, grad, gtau, 1);
+    const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
+    std::vector<float> h(3 * n);
+    if (grad) {
+        if (grad_read_host(m, h.data())) return 1;
+        to_model_layout(m, h, grad, 3);
+    }
+    if (gtau) {
+        if (grad_read_tau_host(m, h.data())) return 1;
+        to_model_layout(m, h, gtau, 2);
+    }
+    return 0;
+}
+
+int seis_grad_read_device(seis_model *m, float *dgrad, float *dgtau) {
+    g_err.clear();
+    if ((dgrad && grad_check(m, false)) || (dgtau && grad_check(m, true))) return 1;
+    const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
+    hipStream_t st = m->ctx->stream;
+    if (grad_on_device(m)) {
+        if ((dgrad || dgtau) && grad_device(m, dgrad, dgtau, 0)) return 1;
+        HIP_TRY(hipStreamSynchronize(st));
+        return 0;
+    }
+    std::vector<float> h(3 * n);
+    if (dgrad) {
+        if (grad_read_host(m, h.data())) return 1;
+        HIP_TRY(hipMemcpyAsync(dgrad, h.data(), 3 * n * 4, hipMemcpyHostToDevice, st));
+        HIP_TRY(hipStreamSynchronize(st));
+    }
+    if (dgtau) {
+        if (grad_read_tau_host(m, h.data())) return 1;
+        HIP_TRY(hipMemcpyAsync(dgtau, h.data(), 2 * n * 4, hipMemcpyHostToDevice, st));
+        HIP_TRY(hipStreamSynchronize(st));
     }
     return 0;
 }

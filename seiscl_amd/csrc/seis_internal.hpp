@@ -453,6 +453,35 @@ struct ResidentAdj2D {
 };
 bool launch_resident_adj2d(ResidentAdj2D &a, int L, int ncu, void *stream, int *err);
 
+// ---------------------------------------------------------------------------
+// Results in the caller's layout (readback.hip).
+// ---------------------------------------------------------------------------
+struct GradOut {
+    Layout lay;
+    const double *g[5];          // accumulators M mu rho tau_p tau_s, padded
+    const void *Ms, *mus;        // moduli of the chain rule, padded (float or double)
+    const float *rho;            // buoyancy dt / (dh rho), padded
+    float dt, dh;
+    double ktau;
+    int param_type, rho_fix;
+    int model;                   // 1: [NZ][NY][NX], 0: [NX][NY][NZ]
+    float *out, *tau;            // [3][N], [2][N]; either may be null
+};
+// f64: Ms and mus are doubles
+void launch_grad_out(const GradOut &a, bool f64, void *stream);
+// seismograms [NT][nout][nrec] (f64: double) -> [nout][NT][nrec]
+void launch_seis_rows(const void *in, bool f64, float *out, int NT, int nout, int nrec,
+                      void *stream);
+// up to kCopyMax arrays in one launch
+constexpr int kCopyMax = 40;
+struct CopyList {
+    int n = 0;
+    const void *src[kCopyMax];
+    void *dst[kCopyMax];
+    size_t bytes[kCopyMax];
+};
+void launch_copy_list(const CopyList &c, void *stream);
+
 // DFT-domain gradient (dft.hip).  The arrays whose spectra are kept:
 // velocities, stresses, then each memory-variable component's L slabs.
 struct DftArrays {

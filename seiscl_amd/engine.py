@@ -202,12 +202,16 @@ class Model:
         sp, s, rp = shot_arrays(src_pos, src, rec_pos)
         nsrc, nrec = sp.shape[0], rp.shape[0]
         NT = self.csts.NT
-        out = np.zeros((len(self.out_names), nrec, NT), dtype=np.float32)
+        out = np.zeros((len(self.out_names), nrec, NT), dtype=np.float32) if raw else None
         check(self.lib.seis_forward_shot(self.handle, nsrc, fptr(sp), fptr(s), nrec,
                                          fptr(rp), fptr(out)))
-        if raw:
-            return out
-        return [np.ascontiguousarray(o.T) for o in out]
+        return out if raw else self._read_nt(nrec)
+
+    def _read_nt(self, nrec: int) -> list:
+        """Seismograms of the last run as (NT, nrec) arrays, one per output."""
+        out = np.empty((len(self.out_names), self.csts.NT, nrec), dtype=np.float32)
+        check(self.lib.seis_shot_read_nt(self.handle, fptr(out)))
+        return list(out)
 
     def bind_shot(self, src_pos, src, rec_pos, init: bool = True):
         """Upload one shot and (init) zero the wavefields (first half of forward)."""
@@ -226,13 +230,11 @@ class Model:
         """Seismograms of the bound shot, (NT, nrec) per output; f64: in
         double, for models running in FP64 (FP16=64)."""
         nrec = self._shot[2].shape[0]
-        dt = np.float64 if f64 else np.float32
-        out = np.zeros((len(self.out_names), nrec, self.csts.NT), dtype=dt)
-        if f64:
-            check(self.lib.seis_shot_read_f64(
-                self.handle, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double))))
-        else:
-            check(self.lib.seis_shot_read(self.handle, fptr(out)))
+        if not f64:
+            return self._read_nt(nrec)
+        out = np.zeros((len(self.out_names), nrec, self.csts.NT), dtype=np.float64)
+        check(self.lib.seis_shot_read_f64(
+            self.handle, out.ctypes.data_as(ctypes.POINTER(ctypes.c_double))))
         return [np.ascontiguousarray(o.T) for o in out]
 
     def read_field(self, name: str) -> np.ndarray:
@@ -272,10 +274,9 @@ class Model:
         adjoint run; returns the seismograms like forward()."""
         self._shot = shot_arrays(src_pos, src, rec_pos)
         sp, s, rp = self._shot
-        out = np.zeros((len(self.out_names), rp.shape[0], self.csts.NT), dtype=np.float32)
         check(self.lib.seis_forward_save(self.handle, sp.shape[0], fptr(sp), fptr(s),
-                                         rp.shape[0], fptr(rp), fptr(out)))
-        return [np.ascontiguousarray(o.T) for o in out]
+                                         rp.shape[0], fptr(rp), None))
+        return self._read_nt(rp.shape[0])
 
     def saved_read(self) -> np.ndarray:
         """The saved forward run of the last forward_save as one host array
@@ -347,17 +348,11 @@ class Model:
     def grad_read(self) -> dict:
         """Accumulated gradients {p0, p1, rho} in the model layout, plus
         {taup, taus} (at fixed wave speeds) for viscoelastic models."""
-        n = int(np.prod(self.shape))
-        g = np.zeros(3 * n, dtype=np.float32)
-        check(self.lib.seis_grad_read(self.handle, fptr(g)))
+        tau = self.csts.L > 0 and self.csts.param_type <= 2
+        g = np.empty((5 if tau else 3,) + tuple(self.shape), dtype=np.float32)
+        check(self.lib.seis_grad_read_model(self.handle, fptr(g[:3]), fptr(g[3:]) if tau else None))
         names = PARAM_NAMES.get(self.csts.param_type, ("vp", "vs", "rho"))
-        out = {nm: from_c_layout(g[q * n:(q + 1) * n], self.shape) for q, nm in enumerate(names)}
-        if self.csts.L > 0 and self.csts.param_type <= 2:
-            t = np.zeros(2 * n, dtype=np.float32)
-            check(self.lib.seis_grad_read_tau(self.handle, fptr(t)))
-            out["taup"] = from_c_layout(t[:n], self.shape)
-            out["taus"] = from_c_layout(t[n:], self.shape)
-        return out
+        return dict(zip(names + (("taup", "taus") if tau else ()), g))
 
     # ---- device-resident variants (torch tensors on the model's GPU) -----
 
