@@ -61,6 +61,108 @@ __device__ __forceinline__ void pml_half(const FDArgs<R> &a, int axis, R &d, R *
     pml(d, psi, cp(a, axis, CBH, kh), cp(a, axis, CAH, kh), cp(a, axis, CKH, kh));
 }
 
+// CPML of the nine velocity derivatives of a 3D stress update, and of the nine
+// stress derivatives of a velocity update: every load before the first store.
+template <typename R>
+__device__ __forceinline__ void cpml_s3d(const FDArgs<R> &a, int z, int y, int x, R &vxx, R &vxy,
+                                         R &vxz, R &vyx, R &vyy, R &vyz, R &vzx, R &vzy, R &vzz) {
+    if (a.abs_type != 1) return;
+    const int NAB = a.nab, NZ = a.g.NZ, NY = a.g.NY, NX = a.g.NX;
+    const bool pz = z > NZ - NAB - 1 || (!a.freesurf && z < NAB);
+    const bool py = y < NAB || y > NY - NAB - 1, px = x < NAB || x > NX - NAB - 1;
+    const bool bot = z > NZ - NAB - 1;
+    const int k = bot ? z - NZ + 2 * NAB : z;
+    const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
+    const int j = y < NAB ? y : y - NY + 2 * NAB;
+    const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
+    const int ii = x < NAB ? x : x - NX + 2 * NAB;
+    const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
+    const long ipz = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
+    const long ipy = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
+    const long ipx = (long)ii * NY * NZ + (long)y * NZ + z;
+    Pml<R> z0, z1, z2, y0, y1, y2, x0, x1, x2;
+    if (pz) {
+        z0 = pml_load(a, a.psi_vx_z + ipz, 2, true, kh);
+        z1 = pml_load(a, a.psi_vy_z + ipz, 2, true, kh);
+        z2 = pml_load(a, a.psi_vz_z + ipz, 2, false, ki);
+    }
+    if (py) {
+        y0 = pml_load(a, a.psi_vx_y + ipy, 1, true, jh);
+        y1 = pml_load(a, a.psi_vy_y + ipy, 1, false, ji);
+        y2 = pml_load(a, a.psi_vz_y + ipy, 1, true, jh);
+    }
+    if (px) {
+        x0 = pml_load(a, a.psi_vx_x + ipx, 0, false, iI);
+        x1 = pml_load(a, a.psi_vy_x + ipx, 0, true, iH);
+        x2 = pml_load(a, a.psi_vz_x + ipx, 0, true, iH);
+    }
+    if (pz) {
+        pml_apply(vxz, a.psi_vx_z + ipz, z0);
+        pml_apply(vyz, a.psi_vy_z + ipz, z1);
+        pml_apply(vzz, a.psi_vz_z + ipz, z2);
+    }
+    if (py) {
+        pml_apply(vxy, a.psi_vx_y + ipy, y0);
+        pml_apply(vyy, a.psi_vy_y + ipy, y1);
+        pml_apply(vzy, a.psi_vz_y + ipy, y2);
+    }
+    if (px) {
+        pml_apply(vxx, a.psi_vx_x + ipx, x0);
+        pml_apply(vyx, a.psi_vy_x + ipx, x1);
+        pml_apply(vzx, a.psi_vz_x + ipx, x2);
+    }
+}
+template <typename R>
+__device__ __forceinline__ void cpml_v3d(const FDArgs<R> &a, int z, int y, int x, R &sxx_x,
+                                         R &sxy_y, R &sxz_z, R &syy_y, R &sxy_x, R &syz_z,
+                                         R &szz_z, R &sxz_x, R &syz_y) {
+    if (a.abs_type != 1) return;
+    const int NAB = a.nab, NZ = a.g.NZ, NY = a.g.NY, NX = a.g.NX;
+    const bool pz = z > NZ - NAB - 1 || (!a.freesurf && z < NAB);
+    const bool py = y < NAB || y > NY - NAB - 1, px = x < NAB || x > NX - NAB - 1;
+    const bool bot = z > NZ - NAB - 1;
+    const int k = bot ? z - NZ + 2 * NAB : z;
+    const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
+    const int j = y < NAB ? y : y - NY + 2 * NAB;
+    const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
+    const int ii = x < NAB ? x : x - NX + 2 * NAB;
+    const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
+    const long ipz = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
+    const long ipy = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
+    const long ipx = (long)ii * NY * NZ + (long)y * NZ + z;
+    Pml<R> z0, z1, z2, y0, y1, y2, x0, x1, x2;
+    if (pz) {
+        z0 = pml_load(a, a.psi_sxz_z + ipz, 2, false, ki);
+        z1 = pml_load(a, a.psi_syz_z + ipz, 2, false, ki);
+        z2 = pml_load(a, a.psi_szz_z + ipz, 2, true, kh);
+    }
+    if (py) {
+        y0 = pml_load(a, a.psi_sxy_y + ipy, 1, false, ji);
+        y1 = pml_load(a, a.psi_syy_y + ipy, 1, true, jh);
+        y2 = pml_load(a, a.psi_syz_y + ipy, 1, false, ji);
+    }
+    if (px) {
+        x0 = pml_load(a, a.psi_sxx_x + ipx, 0, true, iH);
+        x1 = pml_load(a, a.psi_sxy_x + ipx, 0, false, iI);
+        x2 = pml_load(a, a.psi_sxz_x + ipx, 0, false, iI);
+    }
+    if (pz) {
+        pml_apply(sxz_z, a.psi_sxz_z + ipz, z0);
+        pml_apply(syz_z, a.psi_syz_z + ipz, z1);
+        pml_apply(szz_z, a.psi_szz_z + ipz, z2);
+    }
+    if (py) {
+        pml_apply(sxy_y, a.psi_sxy_y + ipy, y0);
+        pml_apply(syy_y, a.psi_syy_y + ipy, y1);
+        pml_apply(syz_y, a.psi_syz_y + ipy, y2);
+    }
+    if (px) {
+        pml_apply(sxx_x, a.psi_sxx_x + ipx, x0);
+        pml_apply(sxy_x, a.psi_sxy_x + ipx, x1);
+        pml_apply(sxz_x, a.psi_sxz_x + ipx, x2);
+    }
+}
+
 // taper factor product of the cell (abs_type 2), applied factor by factor
 template <typename R>
 __device__ __forceinline__ void taper_apply(const FDArgs<R> &a, int z, int y, int x, R *v, int n) {
@@ -149,17 +251,38 @@ __device__ __forceinline__ void grad_mmu_2d(const AdjArgs<R> &A, long i, R sxx, 
     }
 }
 
+// The 3D accumulators of M, mu and tau of a cell as they are before the step:
+// the 3D kernels issue every load of a cell before its first store, which a load
+// that may alias could not pass.  They move 4.5-5 TB/s; at 120 x 128 x 136 the
+// stress step took 98 us with loads after the first stores and takes 93, the
+// velocity step 76.5 and 73; with the history of a viscoelastic gradient in half
+// precision (150 x 130 x 144, L = 2) 190 and 182, 71 and 68.
+struct GradOld {
+    double M = 0, mu = 0, tp = 0, ts = 0;
+};
+template <typename R>
+__device__ __forceinline__ GradOld grad_old(const AdjArgs<R> &A, long i) {
+    GradOld g;
+    g.M = own_ld(A.gM + i);
+    if (!A.rtm) g.mu = own_ld(A.gmu + i);
+    if (A.gtp) {
+        g.tp = own_ld(A.gtp + i);
+        g.ts = own_ld(A.gts + i);
+    }
+    return g;
+}
+
 // The same in 3D (src/update_adjs3D.cl:678-710).  The reference's mu
 // Hessian expression does not compile (one parenthesis too many); here c5
 // weighs the sum of the three squared deviatoric stresses, and the M term is
 // the Hessian's own, as the 2D form with hfix.
 template <typename R>
-__device__ __forceinline__ void grad_mmu_3d(const AdjArgs<R> &A, long i, R sxx, R syy, R szz,
-                                            R sxy, R syz, R sxz, R lsxx, R lsyy, R lszz,
+__device__ __forceinline__ void grad_mmu_3d(const AdjArgs<R> &A, long i, const GradOld &go,
+                                            R sxx, R syy, R szz, R sxy, R syz, R sxz, R lsxx, R lsyy, R lszz,
                                             R lsxy, R lsyz, R lsxz, R lM, R lmu) {
     if (A.rtm) {
         const R dM = (sxx + syy + szz) * (lsxx + lsyy + lszz);
-        own_add(A.gM + i, (double)-dM * A.gscale_s);
+        own_st(A.gM + i, go.M + (double)-dM * A.gscale_s);
         if (A.hM) own_add(A.hM + i, (double)((sxx + syy + szz) * (sxx + syy + szz)) * A.hscale);
         return;
     }
@@ -176,12 +299,12 @@ __device__ __forceinline__ void grad_mmu_3d(const AdjArgs<R> &A, long i, R sxx, 
         own_add(A.gsh[0] + i, (double)(sxz * lsxz) * A.gscale_s);
         own_add(A.gsh[1] + i, (double)(sxy * lsxy) * A.gscale_s);
         own_add(A.gsh[2] + i, (double)(syz * lsyz) * A.gscale_s);
-        own_add(A.gmu + i, (4.0 / 3 * dM - dev) * A.gscale_s);
+        own_st(A.gmu + i, go.mu + (4.0 / 3 * dM - dev) * A.gscale_s);
     } else {
         const double dmu = -c3 * (sxz * lsxz + sxy * lsxy + syz * lsyz) + 4.0 / 3 * dM - dev;
-        own_add(A.gmu + i, dmu * A.gscale_s);
+        own_st(A.gmu + i, go.mu + dmu * A.gscale_s);
     }
-    own_add(A.gM + i, (double)-dM * A.gscale_s);
+    own_st(A.gM + i, go.M + (double)-dM * A.gscale_s);
     if (A.hM) {
         const R dMH = c1 * (sxx + syy + szz) * (sxx + syy + szz);
         const double hmu = c3 * (sxz * sxz + sxy * sxy + syz * syz) - 4.0 / 3 * dMH +
@@ -203,19 +326,19 @@ __device__ __forceinline__ void grad_tau_2d(const AdjArgs<R> &A, long i, R sxx, 
 }
 
 template <typename R>
-__device__ __forceinline__ void grad_tau_3d(const AdjArgs<R> &A, long i, R sxx, R syy, R szz,
-                                            R sxy, R syz, R sxz, R lM, R lmu, R Xp,
+__device__ __forceinline__ void grad_tau_3d(const AdjArgs<R> &A, long i, const GradOld &go,
+                                            R sxx, R syy, R szz, R sxy, R syz, R sxz, R lM, R lmu, R Xp,
                                             const R *X) {
     const R lam = lM - R(2) * lmu;
     const R th = ((sxx + syy) + szz) / (R(3) * lM - R(4) * lmu);
-    own_add(A.gtp + i, (double)(-(th * Xp)) * A.gscale_s);
+    own_st(A.gtp + i, go.tp + (double)(-(th * Xp)) * A.gscale_s);
     if (lmu == R(0)) return;
     const R exx = (sxx - lam * th) / (R(2) * lmu);
     const R eyy = (syy - lam * th) / (R(2) * lmu);
     const R ezz = (szz - lam * th) / (R(2) * lmu);
     const R n3 = (exx * X[0] + eyy * X[1]) + ezz * X[2];
     const R s3 = ((sxy / lmu) * X[3] + (syz / lmu) * X[4]) + (sxz / lmu) * X[5];
-    own_add(A.gts + i, (double)(-(n3 + s3)) * A.gscale_s);
+    own_st(A.gts + i, go.ts + (double)(-(n3 + s3)) * A.gscale_s);
 }
 
 template <typename R, int H>
@@ -353,6 +476,9 @@ __global__ __launch_bounds__(256) void k_adj_s3d(AdjArgs<R> A, int nbz, unsigned
     const R gg = lM, ff = 2.0 * lmu;
     R sxx = own_ld(f.sxx + i), syy = own_ld(f.syy + i), szz = own_ld(f.szz + i);
     R sxy = own_ld(f.sxy + i), syz = own_ld(f.syz + i), sxz = own_ld(f.sxz + i);
+    const R a6[6] = {own_ld(a.sxy + i), own_ld(a.syz + i), own_ld(a.sxz + i),
+                     own_ld(a.sxx + i), own_ld(a.syy + i), own_ld(a.szz + i)};
+    const GradOld go = grad_old(A, i);
     {
         const R vxx = Dm<H>(f.vx, i, sx, hc), vxy = Dp<H>(f.vx, i, sy, hc), vxz = Dp<H>(f.vx, i, 1, hc);
         const R vyx = Dp<H>(f.vy, i, sx, hc), vyy = Dm<H>(f.vy, i, sy, hc), vyz = Dp<H>(f.vy, i, 1, hc);
@@ -376,52 +502,24 @@ __global__ __launch_bounds__(256) void k_adj_s3d(AdjArgs<R> A, int nbz, unsigned
             syz = bnd[7 * n + m];
             sxz = bnd[8 * n + m];
         }
-        own_st(f.sxx + i, sxx);
-        own_st(f.syy + i, syy);
-        own_st(f.szz + i, szz);
-        own_st(f.sxy + i, sxy);
-        own_st(f.syz + i, syz);
-        own_st(f.sxz + i, sxz);
     }
     R vxx = Dm<H>(a.vx, i, sx, hc), vxy = Dp<H>(a.vx, i, sy, hc), vxz = Dp<H>(a.vx, i, 1, hc);
     R vyx = Dp<H>(a.vy, i, sx, hc), vyy = Dm<H>(a.vy, i, sy, hc), vyz = Dp<H>(a.vy, i, 1, hc);
     R vzx = Dp<H>(a.vz, i, sx, hc), vzy = Dp<H>(a.vz, i, sy, hc), vzz = Dm<H>(a.vz, i, 1, hc);
-    const int NAB = a.nab, NZ = g.NZ, NY = g.NY, NX = g.NX;
-    if (a.abs_type == 1) {
-        if (z > NZ - NAB - 1 || (!a.freesurf && z < NAB)) {
-            const bool bot = z > NZ - NAB - 1;
-            const int k = bot ? z - NZ + 2 * NAB : z;
-            const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
-            const long ip = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
-            pml_half(a, 2, vxz, a.psi_vx_z + ip, kh);
-            pml_half(a, 2, vyz, a.psi_vy_z + ip, kh);
-            pml_full(a, 2, vzz, a.psi_vz_z + ip, ki);
-        }
-        if (y < NAB || y > NY - NAB - 1) {
-            const int j = y < NAB ? y : y - NY + 2 * NAB;
-            const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
-            const long ip = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
-            pml_half(a, 1, vxy, a.psi_vx_y + ip, jh);
-            pml_full(a, 1, vyy, a.psi_vy_y + ip, ji);
-            pml_half(a, 1, vzy, a.psi_vz_y + ip, jh);
-        }
-        if (x < NAB || x > NX - NAB - 1) {
-            const int ii = x < NAB ? x : x - NX + 2 * NAB;
-            const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
-            const long ip = (long)ii * NY * NZ + (long)y * NZ + z;
-            pml_full(a, 0, vxx, a.psi_vx_x + ip, iI);
-            pml_half(a, 0, vyx, a.psi_vy_x + ip, iH);
-            pml_half(a, 0, vzx, a.psi_vz_x + ip, iH);
-        }
-    }
+    cpml_s3d(a, z, y, x, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
+    own_st(f.sxx + i, sxx);
+    own_st(f.syy + i, syy);
+    own_st(f.szz + i, szz);
+    own_st(f.sxy + i, sxy);
+    own_st(f.syz + i, syz);
+    own_st(f.sxz + i, sxz);
     const R vxyyx = vxy + vyx, vyzzy = vyz + vzy, vxzzx = vxz + vzx;
     const R vxxyyzz = vxx + vyy + vzz, vyyzz = vyy + vzz, vxxzz = vxx + vzz, vxxyy = vxx + vyy;
     const R lsxy = (fipjp * vxyyx), lsyz = (fjpkp * vyzzy), lsxz = (fipkp * vxzzx);
     const R lsxx = ((gg * vxxyyzz) - (ff * vyyzz));
     const R lsyy = ((gg * vxxyyzz) - (ff * vxxzz));
     const R lszz = ((gg * vxxyyzz) - (ff * vxxyy));
-    R s6[6] = {own_ld(a.sxy + i) + lsxy, own_ld(a.syz + i) + lsyz, own_ld(a.sxz + i) + lsxz,
-               own_ld(a.sxx + i) + lsxx, own_ld(a.syy + i) + lsyy, own_ld(a.szz + i) + lszz};
+    R s6[6] = {a6[0] + lsxy, a6[1] + lsyz, a6[2] + lsxz, a6[3] + lsxx, a6[4] + lsyy, a6[5] + lszz};
     if (a.abs_type == 2) taper_apply(a, z, y, x, s6, 6);
     own_st(a.sxy + i, s6[0]);
     own_st(a.syz + i, s6[1]);
@@ -430,7 +528,7 @@ __global__ __launch_bounds__(256) void k_adj_s3d(AdjArgs<R> A, int nbz, unsigned
     own_st(a.syy + i, s6[4]);
     own_st(a.szz + i, s6[5]);
     // M and mu gradients (src/update_adjs3D.cl:678-710)
-    grad_mmu_3d(A, i, sxx, syy, szz, sxy, syz, sxz, lsxx, lsyy, lszz, lsxy, lsyz, lsxz, lM, lmu);
+    grad_mmu_3d(A, i, go, sxx, syy, szz, sxy, syz, sxz, lsxx, lsyy, lszz, lsxy, lsyz, lsxz, lM, lmu);
 }
 
 template <typename R, int H>
@@ -443,6 +541,8 @@ __global__ __launch_bounds__(256) void k_adj_v3d(AdjArgs<R> A, int nbz, unsigned
     const R *hc = f.hc;
     const R rip = own_ld(f.rip + i), rjp = own_ld(f.rjp + i), rkp = own_ld(f.rkp + i);
     R vx = own_ld(f.vx + i), vy = own_ld(f.vy + i), vz = own_ld(f.vz + i);
+    const R ax = own_ld(a.vx + i), ay = own_ld(a.vy + i), az = own_ld(a.vz + i);
+    const double gr0 = own_ld(A.grho + i);
     {
         const R szz_z = Dp<H>(f.szz, i, 1, hc), sxx_x = Dp<H>(f.sxx, i, sx, hc);
         const R sxz_x = Dm<H>(f.sxz, i, sx, hc), sxz_z = Dm<H>(f.sxz, i, 1, hc);
@@ -460,59 +560,32 @@ __global__ __launch_bounds__(256) void k_adj_v3d(AdjArgs<R> A, int nbz, unsigned
             vy = bnd[n + m];
             vz = bnd[2 * n + m];
         }
-        own_st(f.vx + i, vx);
-        own_st(f.vy + i, vy);
-        own_st(f.vz + i, vz);
     }
     R szz_z = Dp<H>(a.szz, i, 1, hc), sxx_x = Dp<H>(a.sxx, i, sx, hc);
     R sxz_x = Dm<H>(a.sxz, i, sx, hc), sxz_z = Dm<H>(a.sxz, i, 1, hc);
     R syz_y = Dm<H>(a.syz, i, sy, hc), syz_z = Dm<H>(a.syz, i, 1, hc);
     R syy_y = Dp<H>(a.syy, i, sy, hc), sxy_x = Dm<H>(a.sxy, i, sx, hc);
     R sxy_y = Dm<H>(a.sxy, i, sy, hc);
-    const int NAB = a.nab, NZ = g.NZ, NY = g.NY, NX = g.NX;
-    if (a.abs_type == 1) {
-        if (z > NZ - NAB - 1 || (!a.freesurf && z < NAB)) {
-            const bool bot = z > NZ - NAB - 1;
-            const int k = bot ? z - NZ + 2 * NAB : z;
-            const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
-            const long ip = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
-            pml_full(a, 2, sxz_z, a.psi_sxz_z + ip, ki);
-            pml_full(a, 2, syz_z, a.psi_syz_z + ip, ki);
-            pml_half(a, 2, szz_z, a.psi_szz_z + ip, kh);
-        }
-        if (y < NAB || y > NY - NAB - 1) {
-            const int j = y < NAB ? y : y - NY + 2 * NAB;
-            const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
-            const long ip = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
-            pml_full(a, 1, sxy_y, a.psi_sxy_y + ip, ji);
-            pml_half(a, 1, syy_y, a.psi_syy_y + ip, jh);
-            pml_full(a, 1, syz_y, a.psi_syz_y + ip, ji);
-        }
-        if (x < NAB || x > NX - NAB - 1) {
-            const int ii = x < NAB ? x : x - NX + 2 * NAB;
-            const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
-            const long ip = (long)ii * NY * NZ + (long)y * NZ + z;
-            pml_half(a, 0, sxx_x, a.psi_sxx_x + ip, iH);
-            pml_full(a, 0, sxy_x, a.psi_sxy_x + ip, iI);
-            pml_full(a, 0, sxz_x, a.psi_sxz_x + ip, iI);
-        }
-    }
+    cpml_v3d(a, z, y, x, sxx_x, sxy_y, sxz_z, syy_y, sxy_x, syz_z, szz_z, sxz_x, syz_y);
+    own_st(f.vx + i, vx);
+    own_st(f.vy + i, vy);
+    own_st(f.vz + i, vz);
     const R lvx = ((sxx_x + sxy_y + sxz_z) * rip);
     const R lvy = ((syy_y + sxy_x + syz_z) * rjp);
     const R lvz = ((szz_z + sxz_x + syz_y) * rkp);
-    R v3[3] = {own_ld(a.vx + i) + lvx, own_ld(a.vy + i) + lvy, own_ld(a.vz + i) + lvz};
+    R v3[3] = {ax + lvx, ay + lvy, az + lvz};
     if (a.abs_type == 2) taper_apply(a, z, y, x, v3, 3);
     own_st(a.vx + i, v3[0]);
     own_st(a.vy + i, v3[1]);
     own_st(a.vz + i, v3[2]);
     // density gradient (src/update_adjv3D.cl:481)
     if (A.grz) {
-        own_add(A.grho + i, (double)(-vx * lvx));
+        own_st(A.grho + i, gr0 + (double)(-vx * lvx));
         own_add(A.gry + i, (double)(-(vy * lvy)));
         own_add(A.grz + i, (double)(-(vz * lvz)));
     } else {
         const R d = -vx * lvx - vy * lvy - vz * lvz;
-        own_add(A.grho + i, (double)d);
+        own_st(A.grho + i, gr0 + (double)d);
     }
 }
 
@@ -667,48 +740,31 @@ __global__ __launch_bounds__(256) void k_adjh_s3d(AdjArgs<R> A, int nbz, unsigne
     R vxx = Dm<H>(a.vx, i, sx, hc), vxy = Dp<H>(a.vx, i, sy, hc), vxz = Dp<H>(a.vx, i, 1, hc);
     R vyx = Dp<H>(a.vy, i, sx, hc), vyy = Dm<H>(a.vy, i, sy, hc), vyz = Dp<H>(a.vy, i, 1, hc);
     R vzx = Dp<H>(a.vz, i, sx, hc), vzy = Dp<H>(a.vz, i, sy, hc), vzz = Dm<H>(a.vz, i, 1, hc);
-    const int NAB = a.nab, NZ = g.NZ, NY = g.NY, NX = g.NX;
-    if (a.abs_type == 1) {
-        if (z > NZ - NAB - 1 || (!a.freesurf && z < NAB)) {
-            const bool bot = z > NZ - NAB - 1;
-            const int k = bot ? z - NZ + 2 * NAB : z;
-            const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
-            const long ip = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
-            pml_half(a, 2, vxz, a.psi_vx_z + ip, kh);
-            pml_half(a, 2, vyz, a.psi_vy_z + ip, kh);
-            pml_full(a, 2, vzz, a.psi_vz_z + ip, ki);
-        }
-        if (y < NAB || y > NY - NAB - 1) {
-            const int j = y < NAB ? y : y - NY + 2 * NAB;
-            const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
-            const long ip = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
-            pml_half(a, 1, vxy, a.psi_vx_y + ip, jh);
-            pml_full(a, 1, vyy, a.psi_vy_y + ip, ji);
-            pml_half(a, 1, vzy, a.psi_vz_y + ip, jh);
-        }
-        if (x < NAB || x > NX - NAB - 1) {
-            const int ii = x < NAB ? x : x - NX + 2 * NAB;
-            const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
-            const long ip = (long)ii * NY * NZ + (long)y * NZ + z;
-            pml_full(a, 0, vxx, a.psi_vx_x + ip, iI);
-            pml_half(a, 0, vyx, a.psi_vy_x + ip, iH);
-            pml_half(a, 0, vzx, a.psi_vz_x + ip, iH);
-        }
-    }
-    const R vxyyx = vxy + vyx, vyzzy = vyz + vzy, vxzzx = vxz + vzx;
-    const R vxxyyzz = vxx + vyy + vzz, vyyzz = vyy + vzz, vxxzz = vxx + vzz, vxxyy = vxx + vyy;
-    const R DT2 = a.DT2;
+    // every load of the cell before its first store
     const R fipjp = own_ld(a.fipjp + i), fjpkp = own_ld(a.fjpkp + i), fipkp = own_ld(a.fipkp + i);
     const R gg = own_ld(a.cg + i), f = own_ld(a.cf + i), d = own_ld(a.cd + i), e = own_ld(a.ce + i);
     const R dipjp = own_ld(a.dipjp + i), djpkp = own_ld(a.djpkp + i), dipkp = own_ld(a.dipkp + i);
     const long nf = g.nfield;
     R rxy[L], ryz[L], rxz[L], rxx[L], ryy[L], rzz[L];
-    R sumrxy = 0, sumryz = 0, sumrxz = 0, sumrxx = 0, sumryy = 0, sumrzz = 0;
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const long ir = l * nf + i;
         rxy[l] = own_ld(a.rxy + ir); ryz[l] = own_ld(a.ryz + ir); rxz[l] = own_ld(a.rxz + ir);
         rxx[l] = own_ld(a.rxx + ir); ryy[l] = own_ld(a.ryy + ir); rzz[l] = own_ld(a.rzz + ir);
+    }
+    const R a6[6] = {own_ld(a.sxy + i), own_ld(a.syz + i), own_ld(a.sxz + i),
+                     own_ld(a.sxx + i), own_ld(a.syy + i), own_ld(a.szz + i)};
+    const R sxx = hst_own<R, S>(A, 3, i), syy = hst_own<R, S>(A, 4, i), szz = hst_own<R, S>(A, 5, i);
+    const R sxy = hst_own<R, S>(A, 6, i), syz = hst_own<R, S>(A, 7, i), sxz = hst_own<R, S>(A, 8, i);
+    const R lM = own_ld(A.Ms + i), lmu = own_ld(A.mus + i);
+    const GradOld go = grad_old(A, i);
+    cpml_s3d(a, z, y, x, vxx, vxy, vxz, vyx, vyy, vyz, vzx, vzy, vzz);
+    const R vxyyx = vxy + vyx, vyzzy = vyz + vzy, vxzzx = vxz + vzx;
+    const R vxxyyzz = vxx + vyy + vzz, vyyzz = vyy + vzz, vxxzz = vxx + vzz, vxxyy = vxx + vyy;
+    const R DT2 = a.DT2;
+    R sumrxy = 0, sumryz = 0, sumrxz = 0, sumrxx = 0, sumryy = 0, sumrzz = 0;
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
         sumrxy += rxy[l]; sumryz += ryz[l]; sumrxz += rxz[l];
         sumrxx += rxx[l]; sumryy += ryy[l]; sumrzz += rzz[l];
     }
@@ -735,9 +791,9 @@ __global__ __launch_bounds__(256) void k_adjh_s3d(AdjArgs<R> A, int nbz, unsigne
         sumrxy += rxy[l]; sumryz += ryz[l]; sumrxz += rxz[l];
         sumrxx += rxx[l]; sumryy += ryy[l]; sumrzz += rzz[l];
     }
-    R s6[6] = {own_ld(a.sxy + i) + (lsxy + (DT2 * sumrxy)), own_ld(a.syz + i) + (lsyz + (DT2 * sumryz)),
-               own_ld(a.sxz + i) + (lsxz + (DT2 * sumrxz)), own_ld(a.sxx + i) + (lsxx + (DT2 * sumrxx)),
-               own_ld(a.syy + i) + (lsyy + (DT2 * sumryy)), own_ld(a.szz + i) + (lszz + (DT2 * sumrzz))};
+    R s6[6] = {a6[0] + (lsxy + (DT2 * sumrxy)), a6[1] + (lsyz + (DT2 * sumryz)),
+               a6[2] + (lsxz + (DT2 * sumrxz)), a6[3] + (lsxx + (DT2 * sumrxx)),
+               a6[4] + (lsyy + (DT2 * sumryy)), a6[5] + (lszz + (DT2 * sumrzz))};
     if (a.abs_type == 2) taper_apply(a, z, y, x, s6, 6);
     own_st(a.sxy + i, s6[0]);
     own_st(a.syz + i, s6[1]);
@@ -746,10 +802,7 @@ __global__ __launch_bounds__(256) void k_adjh_s3d(AdjArgs<R> A, int nbz, unsigne
     own_st(a.syy + i, s6[4]);
     own_st(a.szz + i, s6[5]);
     // M and mu gradients (src/update_adjs3D.cl:678-710) from the forward state
-    const R sxx = hst_own<R, S>(A, 3, i), syy = hst_own<R, S>(A, 4, i), szz = hst_own<R, S>(A, 5, i);
-    const R sxy = hst_own<R, S>(A, 6, i), syz = hst_own<R, S>(A, 7, i), sxz = hst_own<R, S>(A, 8, i);
-    const R lM = own_ld(A.Ms + i), lmu = own_ld(A.mus + i);
-    grad_mmu_3d(A, i, sxx, syy, szz, sxy, syz, sxz, lsxx, lsyy, lszz, lsxy, lsyz, lsxz, lM, lmu);
+    grad_mmu_3d(A, i, go, sxx, syy, szz, sxy, syz, sxz, lsxx, lsyy, lszz, lsxy, lsyz, lsxz, lM, lmu);
     if (A.gtp) {
         // tau gradients from the whole memory term of the step
         const R vii[3] = {vxx, vyy, vzz};
@@ -764,7 +817,7 @@ __global__ __launch_bounds__(256) void k_adjh_s3d(AdjArgs<R> A, int nbz, unsigne
                                  lsyz + (DT2 * sumryz), Lr, a.DT, A.s0);
         X[5] = tau_part_shear<R>(vxzzx, DT2 * oxz + DT2 * sumrxz, fipkp, dipkp,
                                  lsxz + (DT2 * sumrxz), Lr, a.DT, A.s0);
-        grad_tau_3d(A, i, sxx, syy, szz, sxy, syz, sxz, lM, lmu, Xp, X);
+        grad_tau_3d(A, i, go, sxx, syy, szz, sxy, syz, sxz, lM, lmu, Xp, X);
     }
 }
 
@@ -782,51 +835,26 @@ __global__ __launch_bounds__(256) void k_adjh_v3d(AdjArgs<R> A, int nbz, unsigne
     R syz_y = Dm<H>(a.syz, i, sy, hc), syz_z = Dm<H>(a.syz, i, 1, hc);
     R syy_y = Dp<H>(a.syy, i, sy, hc), sxy_x = Dm<H>(a.sxy, i, sx, hc);
     R sxy_y = Dm<H>(a.sxy, i, sy, hc);
-    const int NAB = a.nab, NZ = g.NZ, NY = g.NY, NX = g.NX;
-    if (a.abs_type == 1) {
-        if (z > NZ - NAB - 1 || (!a.freesurf && z < NAB)) {
-            const bool bot = z > NZ - NAB - 1;
-            const int k = bot ? z - NZ + 2 * NAB : z;
-            const int ki = bot ? 2 * NAB - k : k, kh = bot ? 2 * NAB - 1 - k : k;
-            const long ip = (long)x * NY * 2 * NAB + (long)y * 2 * NAB + k;
-            pml_full(a, 2, sxz_z, a.psi_sxz_z + ip, ki);
-            pml_full(a, 2, syz_z, a.psi_syz_z + ip, ki);
-            pml_half(a, 2, szz_z, a.psi_szz_z + ip, kh);
-        }
-        if (y < NAB || y > NY - NAB - 1) {
-            const int j = y < NAB ? y : y - NY + 2 * NAB;
-            const int ji = y < NAB ? j : 2 * NAB - j, jh = y < NAB ? j : 2 * NAB - 1 - j;
-            const long ip = (long)x * 2 * NAB * NZ + (long)j * NZ + z;
-            pml_full(a, 1, sxy_y, a.psi_sxy_y + ip, ji);
-            pml_half(a, 1, syy_y, a.psi_syy_y + ip, jh);
-            pml_full(a, 1, syz_y, a.psi_syz_y + ip, ji);
-        }
-        if (x < NAB || x > NX - NAB - 1) {
-            const int ii = x < NAB ? x : x - NX + 2 * NAB;
-            const int iI = x < NAB ? ii : 2 * NAB - ii, iH = x < NAB ? ii : 2 * NAB - 1 - ii;
-            const long ip = (long)ii * NY * NZ + (long)y * NZ + z;
-            pml_half(a, 0, sxx_x, a.psi_sxx_x + ip, iH);
-            pml_full(a, 0, sxy_x, a.psi_sxy_x + ip, iI);
-            pml_full(a, 0, sxz_x, a.psi_sxz_x + ip, iI);
-        }
-    }
+    const R ax = own_ld(a.vx + i), ay = own_ld(a.vy + i), az = own_ld(a.vz + i);
+    const R fx = hst_own<R, S>(A, 0, i), fy = hst_own<R, S>(A, 1, i), fz = hst_own<R, S>(A, 2, i);
+    const double gr0 = own_ld(A.grho + i);
+    cpml_v3d(a, z, y, x, sxx_x, sxy_y, sxz_z, syy_y, sxy_x, syz_z, szz_z, sxz_x, syz_y);
     const R lvx = ((sxx_x + sxy_y + sxz_z) * rip);
     const R lvy = ((syy_y + sxy_x + syz_z) * rjp);
     const R lvz = ((szz_z + sxz_x + syz_y) * rkp);
-    R v3[3] = {own_ld(a.vx + i) + lvx, own_ld(a.vy + i) + lvy, own_ld(a.vz + i) + lvz};
+    R v3[3] = {ax + lvx, ay + lvy, az + lvz};
     if (a.abs_type == 2) taper_apply(a, z, y, x, v3, 3);
     own_st(a.vx + i, v3[0]);
     own_st(a.vy + i, v3[1]);
     own_st(a.vz + i, v3[2]);
     // density gradient (src/update_adjv3D.cl:481) from the forward state
     if (A.grz) {
-        own_add(A.grho + i, (double)(-hst_own<R, S>(A, 0, i) * lvx) * A.gscale_v);
-        own_add(A.gry + i, (double)(-(hst_own<R, S>(A, 1, i) * lvy)) * A.gscale_v);
-        own_add(A.grz + i, (double)(-(hst_own<R, S>(A, 2, i) * lvz)) * A.gscale_v);
+        own_st(A.grho + i, gr0 + (double)(-fx * lvx) * A.gscale_v);
+        own_add(A.gry + i, (double)(-(fy * lvy)) * A.gscale_v);
+        own_add(A.grz + i, (double)(-(fz * lvz)) * A.gscale_v);
     } else {
-        const R d = -hst_own<R, S>(A, 0, i) * lvx - hst_own<R, S>(A, 1, i) * lvy -
-                    hst_own<R, S>(A, 2, i) * lvz;
-        own_add(A.grho + i, (double)d * A.gscale_v);
+        const R d = -fx * lvx - fy * lvy - fz * lvz;
+        own_st(A.grho + i, gr0 + (double)d * A.gscale_v);
     }
 }
 
