@@ -337,9 +337,11 @@ int seis_gradient_shot(seis_model *m, int nsrc, const float *src_pos,
 
 /* ---- batched serving (no counterpart in the reference, which runs one    */
 /* shot at a time, src/time_stepping.c:747): up to max_slots modeling jobs, */
-/* each a model with a bound shot, advance together, one launch per kernel  */
-/* class and time step for all of them; a job's results are identical      */
-/* whether it runs alone or in a batch.  2D, FP32, L=0, no free surface.     */
+/* each a model with a bound shot, advance together: large ones one after   */
+/* another, each resident on the chip for the steps of a call, small ones  */
+/* with one launch per pass and time step for all of them; a job's results */
+/* are identical whether it runs alone or in a batch.  2D, FP32, L=0, no    */
+/* free surface.                                                             */
 int seis_batch_create(seis_ctx *ctx, int max_slots, seis_batch **batch);
 int seis_batch_destroy(seis_batch *b);
 /* Add a job (zeroes its wavefields; it starts at step 0); *slot receives   */
@@ -348,7 +350,8 @@ int seis_batch_add(seis_batch *b, seis_model *m, int *slot);
 /* Free a slot (read its seismograms first with seis_shot_read).             */
 int seis_batch_remove(seis_batch *b, int slot);
 /* Advance every job by nsteps steps (jobs at their last step stay idle).    */
-/* Asynchronous: seis_shot_read or seis_ctx_sync wait for it.                */
+/* May return before the steps are made: seis_shot_read or seis_ctx_sync     */
+/* wait for them.                                                            */
 int seis_batch_step(seis_batch *b, int nsteps);
 /* Jobs still stepping and the fewest steps any of them has left.           */
 int seis_batch_status(const seis_batch *b, int *nactive, int *min_left);

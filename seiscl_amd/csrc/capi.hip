@@ -44,8 +44,24 @@ static __device__ __align__(256) unsigned char scratch[SEIS_STATIC_SHOT_BYTES];
 namespace {
 constexpr int kMaxDevices = 64;
 void *g_scratch_dev[kMaxDevices] = {};
-// one resident run at a time on a GPU: two would wait for each other's CUs
-std::mutex g_resident_mu[kMaxDevices];
+// One resident run at a time on a GPU: two would wait for each other's CUs.  run
+// is held for a run, turn while waiting for it, so that two contexts that make
+// one run after another take turns.
+struct ResidentLock {
+    std::mutex turn, run;
+    std::unique_lock<std::mutex> wait() {
+        std::lock_guard<std::mutex> t(turn);
+        return std::unique_lock<std::mutex>(run);
+    }
+    // not held if a run is under way or waited for
+    std::unique_lock<std::mutex> attempt() {
+        std::unique_lock<std::mutex> t(turn, std::try_to_lock);
+        return t ? std::unique_lock<std::mutex>(run, std::try_to_lock)
+                 : std::unique_lock<std::mutex>();
+    }
+} g_resident[kMaxDevices];
+// host words of a context's resident runs in flight together
+constexpr int kResidentFlags = 64;
 std::mutex g_scratch_mu;
 
 // Device address of this GPU's static area (the device must be current).
@@ -104,13 +120,13 @@ struct seis_ctx {
         hipEvent_t freed;           // compute-stream point after the last use
     };
     // workspace of resident 2D runs (fd2d_resident.hip): exchange words and the
-    // run's counters, a host word that a run which gave up sets.  Used under
-    // the GPU's g_resident_mu.
+    // run's counters, host words that runs which gave up set.  Used under the
+    // GPU's g_resident lock.
     struct Resident {
         std::mutex mu;
         void *words = nullptr;
         size_t bytes = 0;
-        int *failed = nullptr;      // pinned host memory
+        int *failed = nullptr;      // [kResidentFlags], pinned host memory
         // CUs; 0: no resident runs (a run gave up: the GPU is shared with another
         // program's kernels)
         int ncu = 0;
@@ -296,8 +312,9 @@ struct seis_model {
     }
 };
 
-// A batch of modeling jobs advanced together, one launch per pass and step
-// for all of them (serving).  Slots hold models with a bound shot.
+// A batch of modeling jobs advanced together (serving): resident runs of one job
+// after another, or one launch per pass and step for all (batch_split).  Slots
+// hold models with a bound shot.
 struct seis_batch {
     seis_ctx *ctx = nullptr;
     int max_slots = 0;
@@ -310,7 +327,7 @@ struct seis_batch {
     BatchTable table{};
     int step = 0;                        // the next batch step to launch
     int maxrec = 0;
-    bool dirty = true;
+    std::vector<int> table_slots;        // the slots of the table; empty: none built
     // host sources of asynchronous copies
     std::vector<BatchSlot> host_slots;
     std::vector<int> host_active;
@@ -713,6 +730,38 @@ bool resident_covers(const seis_model *m, int nsteps) {
     return launch_resident2d(T, m->nd_case, m->ctx->resident.ncu, nullptr, nullptr);
 }
 
+// Sets T's workspace pointers for the next run on the compute stream of m's
+// context and clears what the run needs.  nw: exchange words per cell; flag: the
+// host word that the run sets if it gives up.  The GPU's g_resident is held.
+template <typename Args>
+int resident_workspace(seis_model *m, Args &T, int nw, int flag) {
+    seis_ctx *ctx = m->ctx;
+    seis_ctx::Resident &R = ctx->resident;
+    // words, then the two counters
+    const size_t words = (size_t)nw * m->g.nfield * 8, need = words + 64;
+    if (!R.failed) {
+        void *p = nullptr;
+        HIP_TRY(hipHostMalloc(&p, kResidentFlags * sizeof(int), hipHostMallocMapped));
+        R.failed = (int *)p;
+    }
+    if (need > R.bytes) {
+        if (R.words) ctx->release(R.words);
+        R.words = nullptr;
+        R.bytes = 0;
+        if (ctx->alloc(need, &R.words)) return 1;
+        R.bytes = need;
+    }
+    launch_fill(R.words, need, ctx->stream);
+    R.failed[flag] = 0;
+    void *fd = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&fd, R.failed, 0));
+    T.xch = (unsigned long long *)R.words;
+    T.sync = (int *)((char *)R.words + words);
+    T.patience = R.patience;
+    T.failed = (int *)fd + flag;
+    return 0;
+}
+
 // Makes a resident run on the compute stream and waits for it: launch(T, err)
 // launches it with T's workspace pointers set.  nw: exchange words per cell.
 // *done: 1 if the run was made, 0 if it gave up (the model's state is as before
@@ -723,30 +772,9 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     seis_ctx *ctx = m->ctx;
     seis_ctx::Resident &R = ctx->resident;
     hipStream_t st = ctx->stream;
-    std::lock_guard<std::mutex> lock(g_resident_mu[ctx->device]);
+    const auto lock = g_resident[ctx->device].wait();
     *done = 0;
-    // words, then the two counters
-    const size_t words = (size_t)nw * m->g.nfield * 8, need = words + 64;
-    if (!R.failed) {
-        void *p = nullptr;
-        HIP_TRY(hipHostMalloc(&p, 64, hipHostMallocMapped));
-        R.failed = (int *)p;
-    }
-    if (need > R.bytes) {
-        if (R.words) ctx->release(R.words);
-        R.words = nullptr;
-        R.bytes = 0;
-        if (ctx->alloc(need, &R.words)) return 1;
-        R.bytes = need;
-    }
-    launch_fill(R.words, need, st);
-    *R.failed = 0;
-    void *fd = nullptr;
-    HIP_TRY(hipHostGetDevicePointer(&fd, R.failed, 0));
-    T.xch = (unsigned long long *)R.words;
-    T.sync = (int *)((char *)R.words + words);
-    T.patience = R.patience;
-    T.failed = (int *)fd;
+    if (resident_workspace(m, T, nw, 0)) return 1;
     // (events 0 and 1 time the caller's loop)
     hipEvent_t e0 = pool_event(m, 2), e1 = pool_event(m, 3);
     if (!e0 || !e1) return fail("hipEventCreate failed");
@@ -764,8 +792,9 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     if (ms) HIP_TRY(hipEventElapsedTime(ms, e0, e1));
     return 0;
 }
+int resident_words(const seis_model *m) { return m->nd_case == 22 ? 2 : 4; }
 int resident_forward(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
-    return resident_run(m, T, m->nd_case == 22 ? 2 : 4, done, ms, [&](Resident2D &A, int *e) {
+    return resident_run(m, T, resident_words(m), done, ms, [&](Resident2D &A, int *e) {
         return launch_resident2d(A, m->nd_case, m->ctx->resident.ncu, m->ctx->stream, e);
     });
 }
@@ -3287,7 +3316,7 @@ int seis_batch_add(seis_batch *b, seis_model *m, int *slot) {
     m->in_batch = true;
     b->t[k] = 0;
     b->tmax[k] = sl.tmax;
-    b->dirty = true;
+    b->table_slots.clear();   // a slot in use again is another model
     *slot = k;
     return 0;
 }
@@ -3302,7 +3331,6 @@ int seis_batch_remove(seis_batch *b, int slot) {
     b->model[slot]->done_ev = nullptr;
     b->model[slot]->in_batch = false;
     b->model[slot] = nullptr;
-    b->dirty = true;
     return 0;
 }
 
@@ -3325,16 +3353,15 @@ int seis_batch_slot_left(const seis_batch *b, int slot) {
     return b->tmax[slot] - b->t[slot];
 }
 
-int seis_batch_step(seis_batch *b, int nsteps) {
-    g_err.clear();
+// Steps step0 .. step0 + nsteps - 1 of the given slots with the batch kernels.
+static int batch_passes(seis_batch *b, const std::vector<int> &slots, int step0, int nsteps) {
     hipStream_t st = b->ctx->stream;
-    if (b->dirty) {
+    if (slots != b->table_slots) {
         // rebuild the class tables: slots grouped by (acoustic/elastic, FD order)
         std::map<std::pair<int, int>, std::vector<int>> groups;
         int maxrec = 0;
-        for (int i = 0; i < b->max_slots; ++i) {
+        for (int i : slots) {
             seis_model *m = b->model[i];
-            if (!m) continue;
             groups[{m->nd_case, m->g.H}].push_back(i);
             maxrec = std::max(maxrec, m->shot.nrec);
         }
@@ -3368,18 +3395,118 @@ int seis_batch_step(seis_batch *b, int nsteps) {
         b->table.nblocks = acc;
         b->table.ids = dids;
         b->table.block0 = dtile0;
+        b->table_slots.clear();   // not valid until the copies are queued
         if (!ids.empty())
             HIP_TRY(hipMemcpyAsync(dids, ids.data(), ids.size() * 4, hipMemcpyHostToDevice, st));
         HIP_TRY(hipMemcpyAsync(dtile0, tile0.data(), tile0.size() * 4, hipMemcpyHostToDevice, st));
         b->maxrec = maxrec;
-        b->dirty = false;
+        b->table_slots = slots;
     }
-    int hi = 0;
-    for (int i = 0; i < b->max_slots; ++i)
-        if (b->model[i]) hi = i + 1;
-    launch_batch_steps(b->dslots, hi, b->table, b->maxrec, b->step, nsteps, st);
-    b->step += nsteps;
+    launch_batch_steps(b->dslots, b->table, b->maxrec, step0, nsteps, st);
     HIP_TRY(hipEventRecord(b->table_ev[b->tbuf], st));
+    return 0;
+}
+
+// The slots among live whose next nsteps steps are made as resident runs, one
+// slot after another, and those that share the batch kernels' launches.  The
+// costs are fits (us per step, within 15 %) to both ways on MI355X at 10 thousand
+// to 900 thousand cells, FD order 4 to 12; a resident run adds 60 us, and with the
+// widest tiles its time no longer depends on the grid; the batch kernels' launches
+// take about 19 us however small the slots.  Six slots, batch kernels against
+// resident runs: elastic FD4 200 x 400 25.8 against 22.6, 433 x 1217 62 against 42,
+// FD8 520 x 1400 92 against 98, FD12 433 x 1217 74 against 121, acoustic FD8
+// 600 x 1500 67 against 40; one slot of 100 x 100, elastic FD4: 21 against 3.
+static void batch_split(const seis_batch *b, const std::vector<int> &live, int nsteps,
+                        std::vector<int> &resident, std::vector<int> &passes) {
+    resident.clear();
+    passes.clear();
+    double gain = 19;   // of leaving the passes no slot
+    bool all = true;
+    std::vector<int> slow;
+    for (int i : live) {
+        const seis_model *m = b->model[i];
+        const int n = std::min(nsteps, b->tmax[i] - b->t[i]);
+        if (!resident_covers(m, n)) {
+            all = false;
+            passes.push_back(i);
+            continue;
+        }
+        const int ncu = m->ctx->resident.ncu, H = m->g.H;
+        Resident2D T = resident_args(m, 0, n);
+        launch_resident2d(T, m->nd_case, ncu, nullptr, nullptr);   // the tiles
+        const double cells = (double)m->g.NZ * m->g.NX, cu = cells / ncu;
+        double res, pass;
+        if (m->nd_case == 22) {
+            res = 0.9 + 0.28 * H + (0.83e-3 + 0.08e-3 * H) * cu;
+            pass = 1.1e-5 * cells;
+        } else {
+            res = T.cx + 2 * H > 48 ? 8 + 2 * H : 1.35 + 0.37 * H + (1.45e-3 + 0.33e-3 * H) * cu;
+            pass = (1.35e-5 + 0.1e-5 * H) * cells;
+        }
+        res += 60.0 / n;
+        if (res < pass) {
+            resident.push_back(i);
+        } else {
+            slow.push_back(i);
+            gain += pass - res;
+        }
+    }
+    std::vector<int> &to = all && gain > 0 ? resident : passes;
+    to.insert(to.end(), slow.begin(), slow.end());
+    std::sort(resident.begin(), resident.end());
+    std::sort(passes.begin(), passes.end());
+}
+
+// The next nsteps steps of the given slots as resident runs, waited for.  left:
+// the slots whose run gave up (their state is as before).
+static int batch_resident(seis_batch *b, const std::vector<int> &slots, int nsteps,
+                          std::vector<int> &left) {
+    seis_ctx *ctx = b->ctx;
+    for (size_t k0 = 0; k0 < slots.size(); k0 += kResidentFlags) {
+        const size_t k1 = std::min(slots.size(), k0 + kResidentFlags);
+        for (size_t k = k0; k < k1; ++k) {
+            const int i = slots[k];
+            seis_model *m = b->model[i];
+            Resident2D T = resident_args(m, b->t[i], std::min(nsteps, b->tmax[i] - b->t[i]));
+            T.s = b->host_slots[i].shot;
+            const int flag = (int)(k - k0);
+            if (resident_workspace(m, T, resident_words(m), flag)) return 1;
+            int e = 0;
+            if (!launch_resident2d(T, m->nd_case, ctx->resident.ncu, ctx->stream, &e) ||
+                e != hipSuccess) {
+                (void)hipGetLastError();
+                ctx->resident.failed[flag] = 1;
+            }
+        }
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        for (size_t k = k0; k < k1; ++k)
+            if (((volatile int *)ctx->resident.failed)[k - k0]) left.push_back(slots[k]);
+    }
+    return 0;
+}
+
+int seis_batch_step(seis_batch *b, int nsteps) {
+    g_err.clear();
+    hipStream_t st = b->ctx->stream;
+    std::vector<int> live, resident, left;
+    for (int i = 0; i < b->max_slots; ++i)
+        if (b->model[i] && b->t[i] < b->tmax[i]) live.push_back(i);
+    std::unique_lock<std::mutex> lock;
+    if (b->ctx->resident.ncu) lock = g_resident[b->ctx->device].attempt();
+    if (lock) {
+        std::vector<int> passes;
+        batch_split(b, live, nsteps, resident, passes);
+        live = passes;
+    }
+    if (!live.empty() && nsteps > 0 && batch_passes(b, live, b->step, nsteps)) return 1;
+    if (!resident.empty()) {
+        if (batch_resident(b, resident, nsteps, left)) return 1;
+        if (!left.empty()) {
+            b->ctx->resident.ncu = 0;
+            if (batch_passes(b, left, b->step, nsteps)) return 1;
+        }
+    }
+    b->step += nsteps;
     hipEvent_t ev = b->step_ev[b->step_ev_next++ % b->step_ev.size()];
     HIP_TRY(hipEventRecord(ev, st));
     for (int i = 0; i < b->max_slots; ++i)

@@ -619,27 +619,47 @@ __global__ __launch_bounds__(256) void k_batch_pass(const BatchSlot *__restrict_
     }
 }
 
-__global__ void k_batch_sources(const BatchSlot *slots, int n, int step) {
-    if (threadIdx.x != 0 || (int)blockIdx.x >= n) return;
-    const BatchSlot &S = slots[blockIdx.x];
-    const int t = step - S.start;
-    if (!S.active || t < 0 || t >= S.tmax) return;
-    sources_body<float, float>(S.a, S.nd_case, S.shot, S.NT, t, 1);
-}
-
-__global__ void k_batch_varsout(const BatchSlot *slots, int n, int step) {
-    if ((int)blockIdx.y >= n) return;
-    const BatchSlot &S = slots[blockIdx.y];
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    const int t = step - S.start;
-    if (!S.active || t < 0 || t >= S.tmax || r >= S.shot.nrec) return;
+// Receivers of batch step rec, then the sources of batch step src (either may be
+// negative: none), as k_io.  A slot has gridDim.x blocks of receivers.  (Separate
+// launches for the two took 8.7 us per step, one launch 5.)
+__global__ __launch_bounds__(kIoThreads) void k_batch_io(const BatchSlot *slots, BatchTable tab,
+                                                         int rec, int src) {
+    const BatchSlot &S = slots[tab.ids[blockIdx.y]];
+    if (!S.active) return;
+    const int tr = rec - S.start, ts = src - S.start;
+    const bool dorec = rec >= 0 && tr >= 0 && tr < S.tmax;
+    const bool dosrc = src >= 0 && ts >= 0 && ts < S.tmax && S.shot.nsrc > 0;
+    const ShotDev &s = S.shot;
     OutList o;
     o.n = S.nout;
     for (int q = 0; q < S.nout; ++q) {
         o.code[q] = S.codes[q];
         o.unscale[q] = 1.0f;
     }
-    varsout_body<float, float>(S.a, S.nd_case, S.shot, o, t, r);
+    auto record = [&](int r) { varsout_body<float, float>(S.a, S.nd_case, s, o, tr, r); };
+    const bool one = s.nsrc > kIoSources;   // the first block records all receivers
+    if (dorec && dosrc && !one) {
+        auto on_source = [&](int r) {
+            const int cell = s.rec_cell[r];
+            bool hit = false;
+            for (int k = 0; k < s.nsrc; ++k) hit = hit || s.src_cell[k] == cell;
+            return hit;
+        };
+        const int r0 = blockIdx.x * kIoThreads + threadIdx.x;
+        if (r0 < s.nrec && !on_source(r0)) record(r0);
+        if (blockIdx.x == 0)
+            for (int r = threadIdx.x; r < s.nrec; r += kIoThreads)
+                if (on_source(r)) record(r);
+    } else if (dorec && dosrc) {
+        if (blockIdx.x == 0)
+            for (int r = threadIdx.x; r < s.nrec; r += kIoThreads) record(r);
+    } else if (dorec) {
+        const int r0 = blockIdx.x * kIoThreads + threadIdx.x;
+        if (r0 < s.nrec) record(r0);
+    }
+    if (!dosrc || blockIdx.x != 0) return;
+    __syncthreads();
+    if (threadIdx.x == 0) sources_body<float, float>(S.a, S.nd_case, s, S.NT, ts, 1);
 }
 
 __global__ void k_fill(uint32_t *p, size_t n) {
@@ -762,21 +782,19 @@ void launch_tcounter(int *t, int v, int add, void *stream) {
     hipLaunchKernelGGL(k_tcounter, dim3(1), dim3(64), 0, (hipStream_t)stream, t, v, add);
 }
 
-void launch_batch_steps(const BatchSlot *dslots, int nslots, const BatchTable &tab, int maxrec,
-                        int step0, int nsteps, void *stream) {
+void launch_batch_steps(const BatchSlot *dslots, const BatchTable &tab, int maxrec, int step0,
+                        int nsteps, void *stream) {
     hipStream_t st = (hipStream_t)stream;
-    if (nslots <= 0) return;
+    if (!tab.nblocks || nsteps <= 0) return;
     const dim3 grid(((tab.nblocks + 7) / 8) * 8), blk(BZ, BT);
-    for (int k = 0; k < nsteps; ++k) {
+    const dim3 io(std::max(1, (maxrec + kIoThreads - 1) / kIoThreads), tab.n);
+    for (int k = 0; k <= nsteps; ++k) {
         const int step = step0 + k;
-        hipLaunchKernelGGL(k_batch_sources, dim3(nslots), dim3(64), 0, st, dslots, nslots, step);
-        if (tab.nblocks) {
-            hipLaunchKernelGGL(k_batch_pass<0>, grid, blk, 0, st, dslots, tab, step);
-            hipLaunchKernelGGL(k_batch_pass<1>, grid, blk, 0, st, dslots, tab, step);
-        }
-        if (maxrec > 0)
-            hipLaunchKernelGGL(k_batch_varsout, dim3((maxrec + 255) / 256, nslots), dim3(256), 0,
-                               st, dslots, nslots, step);
+        hipLaunchKernelGGL(k_batch_io, io, dim3(kIoThreads), 0, st, dslots, tab, k ? step - 1 : -1,
+                           k < nsteps ? step : -1);
+        if (k == nsteps) break;
+        hipLaunchKernelGGL(k_batch_pass<0>, grid, blk, 0, st, dslots, tab, step);
+        hipLaunchKernelGGL(k_batch_pass<1>, grid, blk, 0, st, dslots, tab, step);
     }
 }
 

@@ -204,10 +204,11 @@ struct BatchTable {
     const int *ids;          // [n] slot indices (device)
     const unsigned *block0;  // [n+1] first block of each slot (device)
 };
-// Batch steps step0 .. step0+nsteps-1: per step one source launch, one
-// velocity and one stress launch for all slots, one receiver launch.
-void launch_batch_steps(const BatchSlot *dslots, int nslots, const BatchTable &tab, int maxrec,
-                        int step0, int nsteps, void *stream);
+// Batch steps step0 .. step0+nsteps-1 of the table's slots: per step one
+// velocity and one stress launch, and one launch for the receivers and the next
+// step's sources.
+void launch_batch_steps(const BatchSlot *dslots, const BatchTable &tab, int maxrec, int step0,
+                        int nsteps, void *stream);
 
 // ---------------------------------------------------------------------------
 // Gradient by backpropagation (BACK_PROP_TYPE=1).

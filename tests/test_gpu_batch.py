@@ -1,0 +1,65 @@
+"""Batch steps made as resident runs and by the batch kernels, mixed, against the
+same jobs alone, step kernel by step kernel."""
+import numpy as np
+import pytest
+
+from cases import small_case
+
+pytestmark = pytest.mark.gpu
+
+# one large job, small ones of every kind, one with more sources than the
+# receivers' launch compares with, one whose receiver table the resident runs refuse
+JOBS = [dict(ND=2, FDORDER=4, N=(400, 900), NT=90), dict(ND=22, FDORDER=8, N=(70, 90), NT=64),
+        dict(ND=2, FDORDER=8, N=(65, 129), NT=113), dict(ND=22, FDORDER=2, N=(64, 400), NT=40),
+        dict(ND=2, FDORDER=12, N=(90, 120), NT=70), dict(ND=2, FDORDER=4, N=(80, 100), NT=80)]
+
+
+def _job(k, kw):
+    csts, p, (sp, s, rp) = small_case(**kw)
+    if k == 4:
+        sp = np.repeat(sp[:, :1], 17, 1)
+        sp[0] += 10 * np.arange(17)
+        s = np.repeat(s[:, :1], 17, 1)
+        rp[:3, :3] = sp[:3, :3]
+    if k == 5:
+        rp = np.tile(rp, (1, 1100 // rp.shape[1] + 1))
+    rp[:3, 0] = sp[:3, 0]
+    return csts, p, (sp, s, rp)
+
+
+def _alone(ctx, job):
+    from seiscl_amd import Model
+    csts, p, shot = job
+    m = Model(ctx, p, **csts)
+    m.set_profiling(True)
+    out = m.forward(*shot)
+    m.close()
+    return out
+
+
+@pytest.mark.parametrize("chunk", [15, 16, 33, 200])
+@pytest.mark.parametrize("jobs", [[0], [1, 2], [0, 5], [0, 1, 2, 3, 4, 5]], ids=str)
+@pytest.mark.parametrize("wait", [500, 0])
+def test_batch_steps(gpu_ctx, monkeypatch, chunk, jobs, wait):
+    from seiscl_amd import Context, Model
+    from seiscl_amd.engine import Batch
+    jobs = [_job(k, JOBS[k]) for k in jobs]
+    want = [_alone(gpu_ctx, j) for j in jobs]
+    monkeypatch.setenv("SEIS_RESIDENT_WAIT_MS", str(wait))   # 0: every resident run gives up
+    ctx = Context(0)
+    models, b = [], Batch(ctx, 8)
+    for csts, p, shot in jobs:
+        m = Model(ctx, p, **csts)
+        m.bind_shot(*shot)
+        models.append(m)
+        b.add(m)
+        b.step(3)            # later jobs join while the first ones step
+    while b.status()[0]:
+        b.step(chunk)
+    for k, m in enumerate(models):
+        for a, r in zip(m.read_shot(), want[k]):
+            assert np.abs(r).max() > 0 and np.array_equal(a, r)
+        b.remove(k)
+        m.close()
+    b.close()
+    ctx.close()
