@@ -580,6 +580,7 @@ FDArgs<double> as_double(const FDArgs<float> &a) {
     d.freesurf = a.freesurf;
     d.nab = a.nab;
     d.fuse_surface = a.fuse_surface;
+    d.out = a.out;
 #define SEIS_AS_D(f) d.f = (decltype(d.f))(a.f)
     SEIS_AS_D(vx); SEIS_AS_D(vy); SEIS_AS_D(vz); SEIS_AS_D(sxx); SEIS_AS_D(syy); SEIS_AS_D(szz);
     SEIS_AS_D(sxy); SEIS_AS_D(syz); SEIS_AS_D(sxz); SEIS_AS_D(p);
@@ -1995,14 +1996,9 @@ static int forward_save_visco(seis_model *m, float *out) {
         int done = 0;
         if (resident_steps(m, t0, n, true, nullptr, nullptr, nullptr, &done)) return 1;
         if (done) continue;
-        for (int t = t0; t < t0 + n; ++t) {
-            step_sources(m, t, 1, st);
-            step_v(m, st);
-            step_s(m, st);
-            if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
-            step_varsout(m, t, st);
-        }
+        for (int t = t0; t < t0 + n; ++t) step_all(m, t, st);
     }
+    step_io(m, tmax - 1, -1, st);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(st));
     G.saved = true;
@@ -2139,6 +2135,8 @@ struct ViscoAdj {
     int tmin, serial;
     bool half, prof;
     size_t k = 0;               // adjoint steps done (event slots)
+    bool ring = false;          // recompute3d
+    std::vector<std::pair<float *, size_t>> first;   // hf with their bytes
     const MovieOut *mv = nullptr;
 
     // level-l segment [t0, t1), whose starting state is current
@@ -2166,6 +2164,47 @@ struct ViscoAdj {
         return 0;
     }
 
+    // The history of [t0, t1) in 3D: the updates read the wavefields of a step
+    // from its place in the history and store the next step's in the next place,
+    // so only the first step's are copied.  (A copy per step took 35 us, 2.8 million
+    // cells in half precision, beside 162 us for the updates.)  The halo cells of
+    // the history are zero, as the wavefields' are; the image rows are stored by the
+    // stress update.
+    int recompute3d(int t0, int t1) {
+        auto &G = m->grad;
+        hipStream_t st = m->ctx->stream;
+        const size_t slot = hf.size() * fb;
+        struct Keep {
+            seis_model *m;
+            const FDArgs<float> a;
+            const FDArgs<double> ad;
+            ~Keep() {
+                m->a = a;
+                m->ad = ad;
+            }
+        } keep{m, m->a, m->ad};
+        // velocities of step kv and stresses of step ks, new values out bytes on
+        auto at = [&](int kv, int ks, long out) {
+            FDArgs<float> &a = m->a;
+            float **f[] = {&a.vx, &a.vy, &a.vz, &a.sxx, &a.syy, &a.szz, &a.sxy, &a.syz, &a.sxz};
+            for (int q = 0; q < 9; ++q)
+                *f[q] = (float *)((char *)G.hist + (q < 3 ? kv : ks) * slot + q * fb);
+            a.out = out;
+            if (m->prec == P_FP64) m->ad = as_double(a);
+        };
+        if (state_save(first, (char *)G.hist, st)) return 1;
+        for (int k = 0; k < t1 - t0; ++k) {
+            at(k, k, 0);
+            step_sources(m, t0 + k, 1, st);
+            if (t0 + k + 1 == t1) break;   // nothing reads the state after it
+            at(k, k, (long)slot);
+            step_v(m, st);
+            at(k + 1, k, (long)slot);
+            step_s(m, st);
+        }
+        return 0;
+    }
+
     // recompute [t0, t1) keeping every post-source state, then the adjoint
     // steps t1-1 .. max(t0, tmin+1) over them
     int innermost(int t0, int t1) {
@@ -2175,6 +2214,10 @@ struct ViscoAdj {
         const int NT = c.NT, nout = (int)m->outn.size();
         int done = 0;
         if (!mv && resident_steps(m, t0, t1 - t0, false, nullptr, nullptr, G.hist, &done)) return 1;
+        if (!done && ring) {
+            if (recompute3d(t0, t1)) return 1;
+            done = 1;
+        }
         for (int t = t0; t < t1 && !done; ++t) {
             // movie frame: the recomputed forward state at the start of step
             // t, what backpropagation reconstructs after the adjoint step t
@@ -2189,6 +2232,7 @@ struct ViscoAdj {
             }
             cl.n = (int)hf.size();
             launch_copy_list(cl, st);
+            if (t + 1 == t1) break;   // nothing reads the state after it
             step_v(m, st);
             step_s(m, st);
             if (c.freesurf && !m->a.fuse_surface) step_surface(m, st);
@@ -2236,6 +2280,9 @@ static int adjoint_visco(seis_model *m, AdjArgs<R> &A, int serial, const MovieOu
     V.half = m->prec == P_FP16;
     V.prof = m->profiling;
     V.mv = mv;
+    V.ring = m->c.ND == 3 && m->a.fuse_surface && !mv;
+    for (float *f : V.hf) V.first.push_back({f, V.fb});
+    if (V.ring) launch_fill(G.hist, (size_t)P.K[P.L - 1] * V.hf.size() * V.fb, st);
     A.Ms = (const R *)G.Ms;
     A.mus = (const R *)G.mus;
     // with profiling on, events around the two adjoint kernels of every step

@@ -119,6 +119,12 @@ __device__ __forceinline__ bool tile3(int nbz, int NX, int NY, unsigned nb, int 
     return true;
 }
 
+// where an update of field p stores (FDArgs::out)
+template <typename S>
+__device__ __forceinline__ S *out_ptr(S *p, long bytes) {
+    return (S *)((char *)p + bytes);
+}
+
 // Waves per SIMD the velocity update is compiled for: FD orders 2 and 4 fit
 // 80 VGPRs (6 waves instead of 4) without spilling; higher orders need more.
 // (FP64 arithmetic needs twice the registers: no constraint there.)
@@ -218,14 +224,15 @@ void k_v3d(FDArgs<R> a, int nbz, unsigned nb, int yg) {
         if (x < NAB) { vx *= t[x]; vy *= t[x]; vz *= t[x]; }
         if (x > NX - NAB - 1) { vx *= t[NX - x - 1]; vy *= t[NX - x - 1]; vz *= t[NX - x - 1]; }
     }
+    S *vxo = out_ptr(vxp, a.out), *vyo = out_ptr(vyp, a.out), *vzo = out_ptr(vzp, a.out);
     if constexpr (kNTV & 8) {
-        T::stn_(vxp, os, vx);
-        T::stn_(vyp, os, vy);
-        T::stn_(vzp, os, vz);
+        T::stn_(vxo, os, vx);
+        T::stn_(vyo, os, vy);
+        T::stn_(vzo, os, vz);
     } else {
-        T::st(vxp, os, vx);
-        T::st(vyp, os, vy);
-        T::st(vzp, os, vz);
+        T::st(vxo, os, vx);
+        T::st(vyo, os, vy);
+        T::st(vzo, os, vz);
     }
 }
 
@@ -448,8 +455,9 @@ __global__ __launch_bounds__((64 * bys<R, S>())) void k_s3d(FDArgs<R> a, int nbz
             }
         }
     }
-    sts(sxyp, os, sxy); sts(syzp, os, syz); sts(sxzp, os, sxz);
-    sts(sxxp, os, sxx); sts(syyp, os, syy); sts(szzp, os, szz);
+    S *szzo = out_ptr(szzp, a.out), *sxzo = out_ptr(sxzp, a.out), *syzo = out_ptr(syzp, a.out);
+    sts(out_ptr(sxyp, a.out), os, sxy); sts(syzo, os, syz); sts(sxzo, os, sxz);
+    sts(out_ptr(sxxp, a.out), os, sxx); sts(out_ptr(syyp, a.out), os, syy); sts(szzo, os, szz);
     if constexpr (L > 0) {
 #pragma unroll
         for (int l = 0; l < L; ++l) {
@@ -461,10 +469,10 @@ __global__ __launch_bounds__((64 * bys<R, S>())) void k_s3d(FDArgs<R> a, int nbz
     if constexpr (FS) {
         // mirror images above the surface: szz(-m) = -szz(m),
         // sxz(-m) = -sxz(m-1), syz(-m) = -syz(m-1), m = 1..H
-        if (z >= 1 && z <= H) T::st(szzp, os - 2 * z * (unsigned)sizeof(S), -szz);
+        if (z >= 1 && z <= H) T::st(szzo, os - 2 * z * (unsigned)sizeof(S), -szz);
         if (z <= H - 1) {
-            T::st(sxzp, os - (2 * z + 1) * (unsigned)sizeof(S), -sxz);
-            T::st(syzp, os - (2 * z + 1) * (unsigned)sizeof(S), -syz);
+            T::st(sxzo, os - (2 * z + 1) * (unsigned)sizeof(S), -sxz);
+            T::st(syzo, os - (2 * z + 1) * (unsigned)sizeof(S), -syz);
         }
     }
 }

@@ -129,6 +129,9 @@ struct FDArgs {
     R *psi_vx_x, *psi_vy_x, *psi_vz_x, *psi_vx_y, *psi_vy_y, *psi_vz_y,
         *psi_vx_z, *psi_vy_z, *psi_vz_z;
     R *psi_p_x, *psi_p_z;
+    // 3D updates: bytes from a wavefield to the array of its new values (0: in
+    // place)
+    long out;
 };
 
 // Shot description on the device.
