@@ -184,7 +184,15 @@ __device__ __forceinline__ void taper_apply(const FDArgs<R> &a, int z, int y, in
         for (int q = 0; q < n; ++q) v[q] *= t[NX - x - 1];
 }
 
-// lane -> cell, z fastest; 2D uses y = 0
+// lane -> cell, z fastest; 2D uses y = 0.  In 3D the tiles go on along y, or along
+// x within slabs of ABY rows, dealt to the XCDs in turn where their number allows
+// it (fd3d.hip).  Along y, the 2H + 1 planes that the x-differences of NF fields
+// reach pass through an XCD's L2 whole; from 2.25 MB on (half of it) that is
+// slower.  us, stress and velocity step, along y -> along x: 224 x 192 x 208 elastic
+// 394, 312 -> 374, 293 (7.5 MB); 120 x 128 x 136 96, 75 -> 90, 71 (2.5 MB); L = 2 in
+// half precision 224 x 192 x 208 523, 187 -> 503, 172 (3.8 MB), 150 x 130 x 144 182, 67
+// -> 188, 68.5 (2.1 MB).
+template <typename R, int NF>
 __device__ __forceinline__ bool adj_cell(const Layout &g, int nbz, unsigned nb, int &z, int &y,
                                          int &x) {
     unsigned tile;
@@ -195,8 +203,14 @@ __device__ __forceinline__ bool adj_cell(const Layout &g, int nbz, unsigned nb, 
     z = bz * BZ + threadIdx.x;
     if (g.nd == 3) {
         const int nby = (g.NY + ABY - 1) / ABY;
-        y = (r % nby) * ABY + threadIdx.y;
+        int by = r % nby;
         x = r / nby;
+        if (NF * (2 * g.H + 1) * g.sx * (long)sizeof(R) >= 9l << 18) {
+            x = r % g.NX;
+            by = r / g.NX;
+            if (nby % 8 == 0) by = (by % (nby / 8)) * 8 + by / (nby / 8);
+        }
+        y = by * ABY + threadIdx.y;
         return z < g.NZ && y < g.NY && x < g.NX;
     }
     y = 0;
@@ -346,7 +360,7 @@ __global__ __launch_bounds__(256) void k_adj_s2d(AdjArgs<R> A, int nbz, unsigned
     const FDArgs<R> &f = A.f, &a = A.r;
     const Layout &g = f.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 6>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, 0, x), sx = g.sx;
     const R *hc = f.hc;
     const R fipkp = f.muipkp[i], lmu = f.mu[i], lM = f.M[i];
@@ -407,7 +421,7 @@ __global__ __launch_bounds__(256) void k_adj_v2d(AdjArgs<R> A, int nbz, unsigned
     const FDArgs<R> &f = A.f, &a = A.r;
     const Layout &g = f.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 6>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, 0, x), sx = g.sx;
     const R *hc = f.hc;
     const R rip = f.rip[i], rkp = f.rkp[i];
@@ -468,7 +482,7 @@ __global__ __launch_bounds__(256) void k_adj_s3d(AdjArgs<R> A, int nbz, unsigned
     const FDArgs<R> &f = A.f, &a = A.r;
     const Layout &g = f.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 6>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, y, x), sx = g.sx, sy = g.sy;
     const R *hc = f.hc;
     const R fipjp = own_ld(f.muipjp + i), fjpkp = own_ld(f.mujpkp + i), fipkp = own_ld(f.muipkp + i);
@@ -536,7 +550,7 @@ __global__ __launch_bounds__(256) void k_adj_v3d(AdjArgs<R> A, int nbz, unsigned
     const FDArgs<R> &f = A.f, &a = A.r;
     const Layout &g = f.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 6>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, y, x), sx = g.sx, sy = g.sy;
     const R *hc = f.hc;
     const R rip = own_ld(f.rip + i), rjp = own_ld(f.rjp + i), rkp = own_ld(f.rkp + i);
@@ -616,7 +630,7 @@ __global__ __launch_bounds__(256) void k_adjh_s2d(AdjArgs<R> A, int nbz, unsigne
     const FDArgs<R> &a = A.r;
     const Layout &g = a.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 3>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, 0, x), sx = g.sx;
     const R *hc = a.hc;
     R vxx = Dm<H>(a.vx, i, sx, hc), vxz = Dp<H>(a.vx, i, 1, hc);
@@ -691,7 +705,7 @@ __global__ __launch_bounds__(256) void k_adjh_v2d(AdjArgs<R> A, int nbz, unsigne
     const FDArgs<R> &a = A.r;
     const Layout &g = a.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 3>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, 0, x), sx = g.sx;
     const R *hc = a.hc;
     const R rip = a.rip[i], rkp = a.rkp[i];
@@ -734,7 +748,7 @@ __global__ __launch_bounds__(256) void k_adjh_s3d(AdjArgs<R> A, int nbz, unsigne
     const FDArgs<R> &a = A.r;
     const Layout &g = a.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 3>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, y, x), sx = g.sx, sy = g.sy;
     const R *hc = a.hc;
     R vxx = Dm<H>(a.vx, i, sx, hc), vxy = Dp<H>(a.vx, i, sy, hc), vxz = Dp<H>(a.vx, i, 1, hc);
@@ -826,7 +840,7 @@ __global__ __launch_bounds__(256) void k_adjh_v3d(AdjArgs<R> A, int nbz, unsigne
     const FDArgs<R> &a = A.r;
     const Layout &g = a.g;
     int z, y, x;
-    if (!adj_cell(g, nbz, nb, z, y, x)) return;
+    if (!adj_cell<R, 3>(g, nbz, nb, z, y, x)) return;
     const long i = g.idx(z, y, x), sx = g.sx, sy = g.sy;
     const R *hc = a.hc;
     const R rip = own_ld(a.rip + i), rjp = own_ld(a.rjp + i), rkp = own_ld(a.rkp + i);
