@@ -57,7 +57,7 @@
 //                     100 x 100    200 x 400    433 x 1217   600 x 1500
 //   elastic FD4       9.5 -> 2.6   9.8 -> 2.9   13.3 -> 6.4  19.9 -> 13.1
 //   elastic FD8       9.8 -> 3.4   9.8 -> 3.6   15.2 -> 8.3  22.5 -> 17.9
-//   L = 1, FD4        13.3 -> 2.7  14.4 -> 3.0  24.3 -> 6.8  30.3 -> 25.2
+//   L = 1, FD4        13.3 -> 2.7  14.4 -> 3.0  24.3 -> 6.8  not covered
 //   acoustic FD8      8.5 -> 2.4   8.6 -> 2.4   11.5 -> 4.5  14.3 -> 6.1
 // (L = 1 with a free surface.)  Stepping tiles with a halo of 2 H K cells for K
 // steps per launch, without an exchange, costs 10 us to load a 64 x 32 region,
@@ -571,10 +571,10 @@ bool run_resident(Resident2D &a, int ncu, hipStream_t st, int &err) {
 
 // The smallest region that covers the grid.  The lines lie where the next
 // instantiation, or the step kernels, are faster (us per step, resident against
-// step kernels): two Maxwell bodies on 80 columns spill (FD4, 600 x 1500: 32.8
-// against 28.0), one does from FD order 8 on (35.0 against 32.7; FD4 25.2
-// against 30.3), where 16 x 3 columns also lose to 8 x 6 (433 x 1217: 11.2
-// against 10.5; FD4 6.8 against 8.7).
+// step kernels): with one Maxwell body 16 x 3 columns lose to 8 x 6 from FD order 8
+// on (433 x 1217: 11.2 against 10.5; FD4 6.8 against 8.7); on 80 columns a Maxwell
+// body spills, and the step kernels take those grids (600 x 1500, two bodies FD4:
+// 32.8 against 28.0, one body FD8: 35.0 against 32.7).
 template <int H>
 bool dispatch(Resident2D &a, int nd_case, int ncu, hipStream_t st, int &err) {
     if (nd_case == 22)

@@ -480,8 +480,9 @@ class Model:
 
 
 class Batch:
-    """Modeling jobs stepped together (seis_batch): one launch per kernel
-    class and time step advances every job in the batch."""
+    """Modeling jobs stepped together (seis_batch): large jobs one after
+    another, each resident on the chip for the steps of a call, small ones
+    with one launch per pass and time step for all of them."""
 
     def __init__(self, ctx: Context, max_slots: int = 64):
         self.ctx = ctx

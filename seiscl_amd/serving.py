@@ -4,8 +4,8 @@ A request is one modeling job (model, shot, constants) or one gradient job
 (the same plus observed seismograms).  Requests arrive over time.  Modeling
 jobs that the batch kernels cover (2D, FP32, L=0, no free surface) are
 admitted into a batch (seis_batch) while slots and the HBM budget allow;
-every admitted job advances together -- one launch per kernel class and time
-step for the whole batch -- and returns its seismograms as soon as it has run
+every admitted job advances by the same steps at a time -- resident runs of the
+large ones, one launch per pass and time step for the small ones -- and returns its seismograms as soon as it has run
 its last step, freeing its slot for the next arrival.  Gradient jobs, and
 modeling jobs the batch does not cover, run one after another on a second
 context of the same GPU (its own streams), concurrently with the batch.  The
@@ -127,10 +127,10 @@ def serve_batched(ctx: Context, requests, max_slots: int = 48, hbm_budget: float
     time on a second context (run_alone), beside the batch.
 
     Admission to set-up is bounded by HBM (hbm_budget); activation in the
-    batch by the bytes a step touches: ready models join while the active
-    ones' step_bytes stay within cache_budget (three quarters of MI355X's
-    256 MB last-level cache, so that a batch step runs from that cache
-    rather than from HBM), but never fewer than min_slots are active while
+    batch by the bytes a step of the batch kernels touches: ready models join
+    while the active ones' step_bytes stay within cache_budget (three quarters
+    of MI355X's 256 MB last-level cache, so that such a step runs from that
+    cache rather than from HBM), but never fewer than min_slots are active while
     models wait, nor more than max_slots."""
     import queue
     import threading
