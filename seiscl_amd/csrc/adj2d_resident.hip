@@ -619,7 +619,11 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
         __syncthreads();
         sources_out(a.t1 - a.nsteps + 1);
     }
-    if (tid == 0) verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience);
+    if (tid == 0) {
+        const int pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
+        verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience,
+                        pulse < 0 ? nullptr : a.xch + pulse);
+    }
     __syncthreads();
     if (verdict != 1) return;
 

@@ -28,7 +28,8 @@
 // later, after it took the words of the step between from every block it
 // shares a rim with, which those published after they had taken this buffer's.
 // Halo cells of the grid do not change and are not exchanged, the image rows
-// apart.
+// apart; a block whose core holds nothing else takes no words, since it gives
+// none that the others would wait for (resident_tiles.hpp).
 //
 // Every block must be on the chip at once: there is at most one per CU, and the
 // host makes one such run at a time on a GPU.  Kernels of other streams end and
@@ -528,7 +529,11 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     }
 
     // every block's last step is made, or the run has failed
-    if (tid == 0) verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience);
+    if (tid == 0) {
+        const int pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
+        verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience,
+                        pulse < 0 ? nullptr : a.xch + pulse);
+    }
     __syncthreads();
     if (verdict != 1) return;
 

@@ -1,13 +1,13 @@
 // What the resident 2D kernels share: stencils on LDS tiles, CPML, the exchange
-// of rim cells between blocks, the agreement at the end of a run, the tiling.
+// of rim cells between blocks, the agreement at the end of a run.
 // fd2d_resident.hip describes the scheme.
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <type_traits>
 
 #include "fd_common.hpp"
+#include "resident_tiles.hpp"
 #include "seis_internal.hpp"
 
 namespace seis {
@@ -113,40 +113,6 @@ __device__ __forceinline__ void cell_values(const Word *w, float *v) {
     }
 }
 
-// cells of the rim that a block takes from others: z sides, x sides, corners
-constexpr int rim_cells(int H, int CX, int CZ) { return 4 * H * CX + 4 * H * CZ + 4 * H * H; }
-
-// The q-th of them for a block with its region at (rz0, rx0): its LDS cell and
-// its place in the grid, -1 if there is none or it never changes (images: the
-// image rows above the free surface do).
-template <int H, int RZ>
-__device__ __forceinline__ void rim_cell(const Layout &g, int images, int CZ, int CX, int rz0,
-                                         int rx0, int q, int &rl, int &ri) {
-    int lx = 0, lz = 0;
-    bool in = true;
-    const int nz = 4 * H * CX, nx = 4 * H * CZ;
-    if (q < nz) {
-        lz = q % (4 * H);
-        lx = 2 * H + q / (4 * H);
-        if (lz >= 2 * H) lz += CZ;
-    } else if ((q -= nz) < nx) {
-        lz = 2 * H + q % CZ;
-        lx = q / CZ;
-        if (lx >= 2 * H) lx += CX;
-    } else if ((q -= nx) < 4 * H * H) {
-        lz = H + q % (2 * H);
-        lx = H + q / (2 * H);
-        if (lz >= 2 * H) lz += CZ;
-        if (lx >= 2 * H) lx += CX;
-    } else {
-        in = false;
-    }
-    const int zz = rz0 + lz, xx = rx0 + lx;
-    in = in && zz >= (images ? -H : 0) && zz < g.NZ && xx >= 0 && xx < g.NX;
-    rl = lx * RZ + lz;
-    ri = in ? (int)g.idx(zz, 0, xx) : -1;
-}
-
 // Waits for the words of a thread's rim cells and hands their values to
 // put(e, values); false if that took longer than patience.  The first cell is
 // waited for alone and the others are loaded once it is there (they are then, as
@@ -187,17 +153,28 @@ __device__ __forceinline__ bool take_rim(const Word *X, long plane, unsigned tag
 // One thread per block, when its block has made its last step (or given up):
 // 1 once every block of the run has made its last step, 2 if the run failed.
 // sync[0] counts blocks, sync[1] is the run's state, which the last block or one
-// that gave up sets, whichever is first.
+// that gave up sets, whichever is first.  A block of halo cells is here as soon as
+// it has recorded its receivers: it goes on waiting while a neighbour makes steps
+// (pulse: a word of the neighbour's, null for other blocks).
 __device__ __forceinline__ int agree(int *sync, int *failed, int nblocks, int gave_up,
-                                     long long patience) {
+                                     long long patience, const Word *pulse) {
     int st = gave_up ? 2 : 0;
     if (!gave_up) {
         if (__hip_atomic_fetch_add(sync, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == nblocks)
             st = 1;
-        const long long start = wall_clock64();
+        long long start = wall_clock64();
+        Word seen = pulse ? get_word(pulse) : 0;
         while (!st) {
-            st = __hip_atomic_load(sync + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-            if (!st && wall_clock64() - start > patience) st = 2;
+            // (acquired by the exchange below)
+            st = __hip_atomic_load(sync + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (st) break;
+            if (wall_clock64() - start > patience) {
+                const Word now = pulse ? get_word(pulse) : seen;
+                if (now == seen) st = 2;
+                seen = now;
+                start = wall_clock64();
+            }
+            __builtin_amdgcn_s_sleep(4);
         }
     }
     int open = 0;
@@ -206,28 +183,6 @@ __device__ __forceinline__ int agree(int *sync, int *failed, int nblocks, int ga
         st = open;
     if (st == 2) __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     return st;
-}
-
-// Tiles of a grid for one instantiation: nbz x nbx blocks of cores CZ x CX.
-struct Tiling {
-    int nbz = 0, nbx = 0, cz = 0, cx = 0;
-};
-// The fewest rows of tiles, evenly high, then as many columns as the chip has
-// CUs for, but no core narrower than kMinCX.
-constexpr int kMinCX = 4;
-Tiling tiling(const Layout &g, int cols, int ncu) {
-    Tiling t;
-    const int H = g.H, nz = g.NZ + 2 * H, nx = g.NX + 2 * H, czm = 64 - 2 * H, cxm = cols - 2 * H;
-    ncu = ncu / 8 * 8;   // the launch rounds the number of blocks up to 8
-    if (cxm < 1 || ncu < 8) return t;
-    t.nbz = (nz + czm - 1) / czm;
-    t.cz = std::max((nz + t.nbz - 1) / t.nbz, 2 * H + 1);
-    t.nbz = (nz + t.cz - 1) / t.cz;
-    if (t.nbz > ncu) return Tiling();
-    t.cx = std::max(kMinCX, (nx + ncu / t.nbz - 1) / (ncu / t.nbz));
-    if (t.cx > cxm) return Tiling();
-    t.nbx = (nx + t.cx - 1) / t.cx;
-    return t;
 }
 
 }  // namespace

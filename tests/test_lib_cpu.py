@@ -88,6 +88,20 @@ def test_boundary_shell_maps_host(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
+def test_resident_runs_exchange_both_ways(tmp_path):
+    """Blocks of a resident 2D run that wait for another are waited for by it:
+    host code of the library's tiling and rim cells over random grids."""
+    import subprocess
+    here = os.path.dirname(os.path.abspath(__file__))
+    csrc = os.path.join(here, "..", "seiscl_amd", "csrc")
+    exe = str(tmp_path / "tile_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fopenmp", "-I", csrc, "-o", exe,
+                    os.path.join(here, "tile_check.cpp"), os.path.join(csrc, "grad_host.cpp"),
+                    os.path.join(csrc, "setup.cpp")], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
 def test_autograd_module_needs_the_gpu():
     """The autograd wrapper imports without a GPU and fails loudly on use."""
     from seiscl_amd import Context
