@@ -206,6 +206,7 @@ struct seis_model {
     ShotDev shot;
     int shot_nsrc_cap = 0, shot_nrec_cap = 0;
     bool shot_bound = false;
+    bool halo_source = false;        // a source of the bound shot feeds a halo cell
     // timing
     bool profiling = false;
     std::vector<hipEvent_t> evpool;
@@ -1350,6 +1351,7 @@ namespace {
 struct ShotHost {
     std::vector<int> scell, stype, sk, rcell;
     std::vector<float> ss;      // scaled source samples (empty: src as given)
+    bool halo_source = false;   // a source lies on a halo cell
 };
 
 static int shot_host(seis_model *m, int nsrc, const float *src_pos, const float *src, int nrec,
@@ -1363,20 +1365,25 @@ static int shot_host(seis_model *m, int nsrc, const float *src_pos, const float 
     h.sk.assign(nsrc, 0);
     h.rcell.assign(nrec, 0);
     h.ss.clear();
+    h.halo_source = false;
+    bool halo = false;          // of the cell looked at last
     auto cell = [&](const float *p, int &k, int &out) -> int {
         const int i = (int)(p[0] / DH) + H, j = (int)(p[1] / DH) + H;
         k = (int)(p[2] / DH) + H;
         if (k < 0 || k >= g.NZ + 2 * H || (c.ND == 3 && (j < 0 || j >= g.NY + 2 * H)))
             return fail("source or receiver outside the padded grid");
+        halo = false;
         if (i < H || i > g.NX + H - 1) {
             out = -1;   // outside this domain in x: skipped, as the reference does
             return 0;
         }
+        halo = k < H || k >= g.NZ + H || (c.ND == 3 && (j < H || j >= g.NY + H));
         out = (int)g.idx(k - H, c.ND == 3 ? j - H : 0, i - H);
         return 0;
     };
     for (int s = 0; s < nsrc; ++s) {
         if (cell(&src_pos[5 * s], h.sk[s], h.scell[s])) return 1;
+        h.halo_source = h.halo_source || halo;
         h.stype[s] = (int)src_pos[5 * s + 4];
         if (c.ND == 22 && h.stype[s] == 100)
             return fail("explosive sources (type 100) are not defined for ND=22; use type 3");
@@ -1476,6 +1483,7 @@ int seis_shot_bind(seis_model *m, int nsrc, const float *src_pos, const float *s
     m->rcell_host = h.rcell;
     m->recpos_host.assign(rec_pos, rec_pos + (size_t)8 * nrec);
     m->shot_bound = true;
+    m->halo_source = h.halo_source;
     m->grad.saved = false;
     return 0;
 }
@@ -2168,8 +2176,8 @@ struct ViscoAdj {
     // from its place in the history and store the next step's in the next place,
     // so only the first step's are copied.  (A copy per step took 35 us, 2.8 million
     // cells in half precision, beside 162 us for the updates.)  The halo cells of
-    // the history are zero, as the wavefields' are; the image rows are stored by the
-    // stress update.
+    // the history are zero, as the wavefields' are unless a source feeds one (then
+    // states are copied); the image rows are stored by the stress update.
     int recompute3d(int t0, int t1) {
         auto &G = m->grad;
         hipStream_t st = m->ctx->stream;
@@ -2280,7 +2288,7 @@ static int adjoint_visco(seis_model *m, AdjArgs<R> &A, int serial, const MovieOu
     V.half = m->prec == P_FP16;
     V.prof = m->profiling;
     V.mv = mv;
-    V.ring = m->c.ND == 3 && m->a.fuse_surface && !mv;
+    V.ring = m->c.ND == 3 && m->a.fuse_surface && !mv && !m->halo_source;
     for (float *f : V.hf) V.first.push_back({f, V.fb});
     if (V.ring) launch_fill(G.hist, (size_t)P.K[P.L - 1] * V.hf.size() * V.fb, st);
     A.Ms = (const R *)G.Ms;
