@@ -297,7 +297,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
                         const float amp = -1.0f * (a.DT * samp[q]);
                         if (type == 0) lds[5 * FS + c] = lds[5 * FS + c] + amp;
                         else if (type == 2) lds[6 * FS + c] = lds[6 * FS + c] + amp;
-                        else if (type == 3 || type == 100)
+                        else if (type == 1 || type == 3 || type == 100)
                             for (int e = 7; e < 9; ++e)
                                 lds[e * FS + c] =
                                     (float)((double)lds[e * FS + c] + (double)amp / 2.0);

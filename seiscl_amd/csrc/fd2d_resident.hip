@@ -255,8 +255,10 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
                         int f = -1;
                         if (type == 0) f = 0;
                         else if (type == 2) f = 1;
-                        else if (type != 3 && type != 100) continue;
-                        else if (ACOUSTIC) f = 2;
+                        else if (type != 1 && type != 3 && type != 100) continue;
+                        else if (ACOUSTIC) f = type == 1 ? -1 : 2;
+                        // (as sources_body: a y force finds no vy and goes to the
+                        // stresses)
                         if (f >= 0) {
                             B[f * FS + c] = B[f * FS + c] + amp;
                             continue;

@@ -141,6 +141,31 @@ def test_resident_adjoint_equals_steps(gpu_ctx, case):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("case", [
+    dict(ND=2, FDORDER=4, N=(113, 140)), dict(ND=2, FDORDER=8, N=(113, 140), L=1, freesurf=1),
+    dict(ND=22, FDORDER=8, N=(70, 90))], ids=_ids)
+def test_y_forces(gpu_ctx, case):
+    """Source type 1, which has no velocity of its own in 2D, does the same in
+    resident runs and step by step: seismograms, and gradients where there are any."""
+    from seiscl_amd import Model
+    csts, params, (sp, s, rp) = _shot(case)
+    sp[4, :2] = 1
+    cells = rp[[0, 2]].astype(int).T
+    shot = (sp, s, rp[:, np.unique(cells, axis=0, return_index=True)[1]])
+    m = Model(gpu_ctx, params, **csts)
+    runs = []
+    for prof in (False, True):
+        m.set_profiling(prof)
+        r = list(m.forward(*shot))
+        if case["ND"] == 2:
+            g, f = _gradient(m, shot)
+            r += list(g.values()) + f
+        runs.append(r)
+    m.close()
+    for a, b in zip(*runs):
+        assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
 def test_run_that_gives_up_is_made_by_steps(gpu_ctx, monkeypatch):
     """Blocks that do not wait at all: the run ends, the model's state is as
     before it, and the step kernels make the steps."""
