@@ -108,6 +108,15 @@ int seis_ctx_create(int device_ordinal, seis_ctx **ctx);
 int seis_ctx_destroy(seis_ctx *ctx);
 int seis_ctx_sync(seis_ctx *ctx);                   /* WAITQUEUE (src/F.h:634)  */
 size_t seis_ctx_footprint(const seis_ctx *ctx);     /* device bytes allocated   */
+/* 2D runs of the context that stayed on the chip for all their steps (one    */
+/* launch): made[2] and gave_up[2], each forward then adjoint (either may be  */
+/* NULL).  A run gives up when one of its blocks waits for another for more  */
+/* than SEIS_RESIDENT_WAIT_MS milliseconds (environment, read by              */
+/* seis_ctx_create, default 500), because other kernels hold part of the GPU. */
+/* Its steps are then made by the step kernels, with the same results, as are */
+/* those of later runs for a hundred times as long.  No counterpart in the    */
+/* reference.                                                                  */
+int seis_ctx_resident_runs(const seis_ctx *ctx, long long *made, long long *gave_up);
 
 /* ---- buffers: replace clbuf_create / clbuf_send / clbuf_read              */
 /* (src/clbuf.c:23-281).  Transfers are ordered on the compute stream.        */

@@ -67,6 +67,8 @@ SIGNATURES = [
     ("seis_ctx_destroy", _I, [_P]),
     ("seis_ctx_sync", _I, [_P]),
     ("seis_ctx_footprint", ctypes.c_size_t, [_P]),
+    ("seis_ctx_resident_runs", _I, [_P, ctypes.POINTER(ctypes.c_longlong),
+                                    ctypes.POINTER(ctypes.c_longlong)]),
     ("seis_buf_create", _I, [_P, ctypes.c_size_t, ctypes.POINTER(_P)]),
     ("seis_buf_free", _I, [_P, _P]),
     ("seis_buf_send", _I, [_P, _P, _P, ctypes.c_size_t]),

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -123,15 +124,21 @@ struct seis_ctx {
     // run's counters, host words that runs which gave up set.  Used under the
     // GPU's g_resident lock.
     struct Resident {
-        std::mutex mu;
         void *words = nullptr;
         size_t bytes = 0;
         int *failed = nullptr;      // [kResidentFlags], pinned host memory
-        // CUs; 0: no resident runs (a run gave up: the GPU is shared with another
-        // program's kernels)
-        int ncu = 0;
+        int ncu = 0;                // CUs
         // longest wait of a block for another, in wall_clock64 ticks
         long long patience = 0;
+        RunRest rest;
+        // forward, adjoint
+        std::atomic<long long> made[2] = {{0}, {0}}, gave_up[2] = {{0}, {0}};
+
+        bool open() const { return ncu && rest.over(); }
+        void count(bool adjoint, bool done) {
+            ++(done ? made : gave_up)[adjoint];
+            if (!done) rest.begin();
+        }
     } resident;
     std::map<void *, size_t> allocs;          // live block -> requested bytes
     std::map<void *, size_t> caps;            // every block -> capacity
@@ -724,7 +731,7 @@ Resident2D resident_args(const seis_model *m, int t0, int nsteps) {
 // wavefields in 32 bits, up to two Maxwell bodies, source and receiver tables
 // that fit a block's lists, a grid that fits the CUs.
 bool resident_covers(const seis_model *m, int nsteps) {
-    if (m->nd_case == 3 || (m->prec != P_FP32 && m->prec != P_SCALED) || !m->ctx->resident.ncu ||
+    if (m->nd_case == 3 || (m->prec != P_FP32 && m->prec != P_SCALED) || !m->ctx->resident.open() ||
         m->c.L > (m->nd_case == 22 ? 0 : 2) || nsteps < kResidentMinSteps ||
         m->shot.nsrc > kResidentMaxSrc || m->shot.nrec > kResidentMaxRec)
         return false;
@@ -771,6 +778,7 @@ int resident_workspace(seis_model *m, Args &T, int nw, int flag) {
 // wanted.
 template <typename Args, typename F>
 int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launch) {
+    constexpr bool adjoint = std::is_same<Args, ResidentAdj2D>::value;
     seis_ctx *ctx = m->ctx;
     seis_ctx::Resident &R = ctx->resident;
     hipStream_t st = ctx->stream;
@@ -784,13 +792,13 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     int e = 0;
     if (!launch(T, &e) || e != hipSuccess) {
         (void)hipGetLastError();
-        R.ncu = 0;
+        R.count(adjoint, false);
         return 0;
     }
     HIP_TRY(hipEventRecord(e1, st));
     HIP_TRY(hipEventSynchronize(e1));
     *done = !*(volatile int *)R.failed;
-    if (!*done) R.ncu = 0;
+    R.count(adjoint, *done);
     if (ms) HIP_TRY(hipEventElapsedTime(ms, e0, e1));
     return 0;
 }
@@ -1140,18 +1148,28 @@ int seis_ctx_create(int device_ordinal, seis_ctx **out) {
     HIP_TRY(hipStreamCreateWithFlags(&ctx->xfer, hipStreamNonBlocking));
     // SEIS_RESIDENT_WAIT_MS: longest wait of a block of a resident run for
     // another block (default 500); a run that waits longer is made again by the
-    // step kernels, as are all later ones of the context
+    // step kernels, as are the later ones for a hundred times as long
     int ncu = 0, khz = 0;
     const char *wait = getenv("SEIS_RESIDENT_WAIT_MS");
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_ordinal) != hipSuccess ||
         khz <= 0)
         khz = 100000;
-    ctx->resident.patience = (long long)(wait && *wait ? std::max(0, atoi(wait)) : 500) * khz;
+    const int wait_ms = wait && *wait ? std::max(0, atoi(wait)) : 500;
+    ctx->resident.patience = (long long)wait_ms * khz;
+    ctx->resident.rest.set_wait(wait_ms);
     if (device_ordinal < kMaxDevices &&
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device_ordinal) ==
             hipSuccess)
         ctx->resident.ncu = ncu;
     *out = ctx.release();
+    return 0;
+}
+
+int seis_ctx_resident_runs(const seis_ctx *ctx, long long *made, long long *gave_up) {
+    for (int k = 0; k < 2; ++k) {
+        if (made) made[k] = ctx->resident.made[k];
+        if (gave_up) gave_up[k] = ctx->resident.gave_up[k];
+    }
     return 0;
 }
 
@@ -2062,7 +2080,7 @@ static int resident_adjoint(seis_model *m, const AdjArgs<R> &A, int t1, int n, i
         auto &G = m->grad;
         const seis_csts &c = m->c;
         const int ncu = m->ctx->resident.ncu, nout = (int)m->out_codes.size();
-        if (c.ND != 2 || m->prec == P_FP16 || m->profiling || !ncu || c.L > 2 ||
+        if (c.ND != 2 || m->prec == P_FP16 || m->profiling || !m->ctx->resident.open() || c.L > 2 ||
             c.abs_type == 2 || A.rtm || A.hM || A.grz || serial || nout > 6 ||
             n < kResidentMinSteps || m->shot.nsrc > kResidentMaxSrc ||
             m->shot.nrec > kResidentMaxRec)
@@ -3534,8 +3552,11 @@ static int batch_resident(seis_batch *b, const std::vector<int> &slots, int nste
             }
         }
         HIP_TRY(hipStreamSynchronize(ctx->stream));
-        for (size_t k = k0; k < k1; ++k)
-            if (((volatile int *)ctx->resident.failed)[k - k0]) left.push_back(slots[k]);
+        for (size_t k = k0; k < k1; ++k) {
+            const bool done = !((volatile int *)ctx->resident.failed)[k - k0];
+            ctx->resident.count(false, done);
+            if (!done) left.push_back(slots[k]);
+        }
     }
     return 0;
 }
@@ -3547,7 +3568,7 @@ int seis_batch_step(seis_batch *b, int nsteps) {
     for (int i = 0; i < b->max_slots; ++i)
         if (b->model[i] && b->t[i] < b->tmax[i]) live.push_back(i);
     std::unique_lock<std::mutex> lock;
-    if (b->ctx->resident.ncu) lock = g_resident[b->ctx->device].attempt();
+    if (b->ctx->resident.open()) lock = g_resident[b->ctx->device].attempt();
     if (lock) {
         std::vector<int> passes;
         batch_split(b, live, nsteps, resident, passes);
@@ -3556,10 +3577,7 @@ int seis_batch_step(seis_batch *b, int nsteps) {
     if (!live.empty() && nsteps > 0 && batch_passes(b, live, b->step, nsteps)) return 1;
     if (!resident.empty()) {
         if (batch_resident(b, resident, nsteps, left)) return 1;
-        if (!left.empty()) {
-            b->ctx->resident.ncu = 0;
-            if (batch_passes(b, left, b->step, nsteps)) return 1;
-        }
+        if (!left.empty() && batch_passes(b, left, b->step, nsteps)) return 1;
     }
     b->step += nsteps;
     hipEvent_t ev = b->step_ev[b->step_ev_next++ % b->step_ev.size()];

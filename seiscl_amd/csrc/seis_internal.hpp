@@ -10,6 +10,8 @@
 // sy = 0.  CPML memory arrays keep the compact strip layout of the
 // reference (src/update_v3D.cl:23-31).
 #pragma once
+#include <atomic>
+#include <chrono>
 #include <cstddef>
 #include <cstdint>
 #include <string>
@@ -419,6 +421,25 @@ struct Resident2D {
     int cz, cx, nbz;
     unsigned ntile;
 };
+// After a run that gave up a context makes no others for a hundred times the wait:
+// where another program's kernels hold CUs for good, trying again costs one
+// percent, and a stall that passes costs a while.  (Read and begun by any thread.)
+class RunRest {
+public:
+    using clock = std::chrono::steady_clock;
+    void set_wait(int ms) { length_ = std::chrono::milliseconds(100) * ms; }
+    void begin(clock::time_point now = clock::now()) {
+        until_ = (now + length_).time_since_epoch().count();
+    }
+    bool over(clock::time_point now = clock::now()) const {
+        return now.time_since_epoch().count() >= until_.load();
+    }
+
+private:
+    clock::duration length_{};
+    std::atomic<clock::rep> until_{clock::duration::min().count()};
+};
+
 // Steps t0 .. t0 + nsteps - 1 on ncu CUs; false: the grid does not fit.  err:
 // the launch's hipError_t.  stream null: nothing is launched.
 bool launch_resident2d(Resident2D &a, int nd_case, int ncu, void *stream, int *err);

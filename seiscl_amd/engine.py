@@ -149,6 +149,13 @@ class Context:
     def footprint(self) -> int:
         return int(self.lib.seis_ctx_footprint(self.handle))
 
+    def resident_runs(self) -> dict:
+        """2D runs that stayed on the chip and such that gave up (and were made
+        by the step kernels), as (forward, adjoint) pairs."""
+        made, gave_up = (ctypes.c_longlong * 2)(), (ctypes.c_longlong * 2)()
+        check(self.lib.seis_ctx_resident_runs(self.handle, made, gave_up))
+        return dict(made=tuple(made), gave_up=tuple(gave_up))
+
     def sync(self):
         check(self.lib.seis_ctx_sync(self.handle))
 

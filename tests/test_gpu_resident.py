@@ -179,12 +179,14 @@ def test_run_that_gives_up_is_made_by_steps(gpu_ctx, monkeypatch):
     monkeypatch.setenv("SEIS_RESIDENT_WAIT_MS", "0")
     ctx = Context(0)
     m = Model(ctx, params, **csts)
-    for _ in range(2):
-        got, fields = m.forward(*shot), _state(m, 2)
-        for a, b in zip(got + fields, ref + rfields):
-            assert np.array_equal(a, b)
+    got = [m.forward(*shot) + _state(m, 2) for _ in range(2)]
+    runs = ctx.resident_runs()
     m.close()
     ctx.close()
+    for k in range(2):
+        for a, b in zip(got[k], ref + rfields):
+            assert np.array_equal(a, b)
+    assert runs == dict(made=(0, 0), gave_up=(2, 0))
 
 
 @pytest.mark.parametrize("L", [0, 1])

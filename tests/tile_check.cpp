@@ -3,7 +3,8 @@
 // of the step between from every block whose rim the word lies in.  That holds if
 // block A takes cells of block B exactly if B takes cells of A, and every word
 // that is waited for is one that its owner publishes (the outer 2H cells of its
-// core).  Blocks of halo cells neither take nor are waited for.  Built and run by test_lib_cpu.py.
+// core).  Blocks of halo cells neither take nor are waited for.  And the pause
+// after a run that gave up (seis::RunRest).  Built and run by test_lib_cpu.py.
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -80,7 +81,23 @@ static void sweep(std::mt19937 &rng) {
     check<H>(211, 397, 16, 256, 1);
 }
 
+// The pause after a run that gave up: a hundred waits, then runs again.
+static void check_rest() {
+    using namespace std::chrono;
+    const auto t = seis::RunRest::clock::now();
+    seis::RunRest r;
+    if (!r.over(t)) ++bad;
+    r.set_wait(5);
+    if (!r.over(t)) ++bad;
+    r.begin(t);
+    if (r.over(t) || r.over(t + milliseconds(499)) || !r.over(t + milliseconds(500))) ++bad;
+    r.set_wait(0);
+    r.begin(t);
+    if (!r.over(t)) ++bad;
+}
+
 int main() {
+    check_rest();
     std::mt19937 rng(7);
     sweep<1>(rng);
     sweep<2>(rng);
