@@ -476,7 +476,8 @@ class Model:
 
     def close(self):
         if getattr(self, "handle", None):
-            self.lib.seis_model_destroy(self.handle)
+            if self.ctx.handle:    # a closed context has taken its memory with it
+                self.lib.seis_model_destroy(self.handle)
             self.handle = None
 
     def __del__(self):
@@ -522,7 +523,8 @@ class Batch:
 
     def close(self):
         if getattr(self, "handle", None):
-            self.lib.seis_batch_destroy(self.handle)
+            if self.ctx.handle:    # a closed context has taken its memory with it
+                self.lib.seis_batch_destroy(self.handle)
             self.handle = None
 
     def __del__(self):

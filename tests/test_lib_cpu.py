@@ -102,6 +102,31 @@ def test_resident_runs_exchange_both_ways(tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
+def test_close_after_the_context():
+    """A model or batch closed (or collected) after its context is not handed to
+    the library, whose context, and with it all device memory, is gone."""
+    from seiscl_amd.engine import Batch, Context, Model
+    calls = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda h: calls.append((name, h))
+
+    for cls, name in ((Model, "seis_model_destroy"), (Batch, "seis_batch_destroy")):
+        for alive in (True, False):
+            ctx = Context.__new__(Context)
+            ctx.lib, ctx.handle = Lib(), "ctx"
+            obj = cls.__new__(cls)
+            obj.lib, obj.ctx, obj.handle = ctx.lib, ctx, "obj"
+            calls.clear()
+            if not alive:
+                ctx.close()
+            obj.close()
+            obj.close()
+            assert ((name, "obj") in calls) == alive and obj.handle is None
+            assert calls.count((name, "obj")) == int(alive)
+
+
 def test_autograd_module_needs_the_gpu():
     """The autograd wrapper imports without a GPU and fails loudly on use."""
     from seiscl_amd import Context
