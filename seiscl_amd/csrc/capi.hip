@@ -727,13 +727,14 @@ Resident2D resident_args(const seis_model *m, int t0, int nsteps) {
     return T;
 }
 
-// Whether a run of nsteps steps of the bound shot can stay on the chip: 2D,
+// Whether a run of nsteps steps of shot s (the bound one, or a batch slot's, which
+// stays as it was when the model is bound to another) can stay on the chip: 2D,
 // wavefields in 32 bits, up to two Maxwell bodies, source and receiver tables
 // that fit a block's lists, a grid that fits the CUs.
-bool resident_covers(const seis_model *m, int nsteps) {
+bool resident_covers(const seis_model *m, const ShotDev &s, int nsteps) {
     if (m->nd_case == 3 || (m->prec != P_FP32 && m->prec != P_SCALED) || !m->ctx->resident.open() ||
         m->c.L > (m->nd_case == 22 ? 0 : 2) || nsteps < kResidentMinSteps ||
-        m->shot.nsrc > kResidentMaxSrc || m->shot.nrec > kResidentMaxRec)
+        s.nsrc > kResidentMaxSrc || s.nrec > kResidentMaxRec)
         return false;
     Resident2D T = resident_args(m, 0, nsteps);
     return launch_resident2d(T, m->nd_case, m->ctx->resident.ncu, nullptr, nullptr);
@@ -815,7 +816,7 @@ int resident_forward(seis_model *m, Resident2D &T, int *done, float *ms = nullpt
 int resident_steps(seis_model *m, int t0, int n, bool rec, float *bnd, const Shell *sh,
                    float *hist, int *done) {
     *done = 0;
-    if (m->profiling || !resident_covers(m, n)) return 0;
+    if (m->profiling || !resident_covers(m, m->shot, n)) return 0;
     Resident2D T = resident_args(m, t0, n);
     if (!rec) T.s.nrec = 0;
     T.bnd = bnd;
@@ -1622,7 +1623,7 @@ int seis_run_steps(seis_model *m, int t0, int nsteps) {
     if (!e0 || !e1) return fail("hipEventCreate failed");
     const bool prof = m->profiling;
     if (prof && !pool_event(m, 2 + 4 * (size_t)nsteps)) return fail("hipEventCreate failed");
-    if (!prof && resident_covers(m, nsteps)) {
+    if (!prof && resident_covers(m, m->shot, nsteps)) {
         Resident2D T = resident_args(m, t0, nsteps);
         int done = 0;
         float ms = 0;
@@ -3499,7 +3500,7 @@ static void batch_split(const seis_batch *b, const std::vector<int> &live, int n
     for (int i : live) {
         const seis_model *m = b->model[i];
         const int n = std::min(nsteps, b->tmax[i] - b->t[i]);
-        if (!resident_covers(m, n)) {
+        if (!resident_covers(m, b->host_slots[i].shot, n)) {
             all = false;
             passes.push_back(i);
             continue;

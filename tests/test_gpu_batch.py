@@ -74,3 +74,28 @@ def test_batch_steps(gpu_ctx, monkeypatch, chunk, jobs, wait):
     assert (runs["made"][0] > 0) == (resident and wait > 0)
     assert (runs["gave_up"][0] > 0) == (resident and wait == 0)
     assert runs["made"][1] == runs["gave_up"][1] == 0
+
+
+def test_model_bound_again_in_the_batch(gpu_ctx):
+    """A slot steps the shot it was added with: 1100 receivers stay with the batch
+    kernels also when the model is bound to a few of them."""
+    from seiscl_amd import Model
+    from seiscl_amd.engine import Batch
+    csts, p, (sp, s, rp) = small_case(ND=2, FDORDER=4, N=(80, 100), NT=80)
+    rp = np.tile(rp, (1, 1100 // rp.shape[1] + 1))
+    m, b = Model(gpu_ctx, p, **csts), Batch(gpu_ctx, 2)
+    before = gpu_ctx.resident_runs()
+    m.bind_shot(sp, s, rp)
+    b.add(m)
+    m.bind_shot(sp, s, rp[:, :7], init=False)
+    b.step(80)
+    gpu_ctx.sync()
+    field = m.read_field("vx")
+    after = gpu_ctx.resident_runs()
+    b.close()
+    m.set_profiling(True)
+    m.forward(sp, s, rp)
+    want = m.read_field("vx")
+    m.close()
+    assert before == after
+    assert np.abs(want).max() > 0 and np.array_equal(field, want)
