@@ -114,8 +114,10 @@ size_t seis_ctx_footprint(const seis_ctx *ctx);     /* device bytes allocated   
 /* than SEIS_RESIDENT_WAIT_MS milliseconds (environment, read by              */
 /* seis_ctx_create, default 500), because other kernels hold part of the GPU. */
 /* Its steps are then made by the step kernels, with the same results, as are */
-/* those of later runs for a hundred times as long.  No counterpart in the    */
-/* reference.                                                                  */
+/* those of later runs for a hundred times as long.  While another process    */
+/* makes such a run on the GPU (a lock on /tmp/seiscl_amd-resident-<PCI bus    */
+/* id>.lock), this one's steps are made by the step kernels at once and count */
+/* as neither.  No counterpart in the reference.                              */
 int seis_ctx_resident_runs(const seis_ctx *ctx, long long *made, long long *gave_up);
 
 /* ---- buffers: replace clbuf_create / clbuf_send / clbuf_read              */

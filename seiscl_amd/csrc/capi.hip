@@ -2,10 +2,13 @@
 // time loop.  Replaces the reference's Init_OpenCL / clprogram / clbuf layer
 // and the forward half of time_stepping (src/time_stepping.c:553-848).
 #include <hip/hip_fp16.h>
+#include <fcntl.h>
 #include <hip/hip_runtime.h>
+#include <sys/file.h>
 
 #include <algorithm>
 #include <atomic>
+#include <cerrno>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -13,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "seis_internal.hpp"
@@ -47,18 +51,63 @@ constexpr int kMaxDevices = 64;
 void *g_scratch_dev[kMaxDevices] = {};
 // One resident run at a time on a GPU: two would wait for each other's CUs.  run
 // is held for a run, turn while waiting for it, so that two contexts that make
-// one run after another take turns.
+// one run after another take turns.  Between processes a file lock: while another
+// process makes a run, this one's steps are the step kernels'.
 struct ResidentLock {
     std::mutex turn, run;
-    std::unique_lock<std::mutex> wait() {
+    std::once_flag named;
+    std::string path;                // of the lock file, set with the GPU's first context
+    int fd = -1;
+    class Held {
+    public:
+        Held() = default;
+        Held(std::unique_lock<std::mutex> l, ResidentLock &r) : lock_(std::move(l)) {
+            if (!lock_) return;
+            file_ = r.file();
+            if (file_ >= 0 && flock(file_, LOCK_EX | LOCK_NB)) {
+                file_ = -1;
+                if (errno == EWOULDBLOCK) lock_.unlock();
+            }
+        }
+        Held(Held &&o) noexcept : lock_(std::move(o.lock_)), file_(std::exchange(o.file_, -1)) {}
+        Held &operator=(Held &&o) noexcept {
+            std::swap(lock_, o.lock_);
+            std::swap(file_, o.file_);
+            return *this;
+        }
+        // (the file's lock goes first: it is the process's, not the thread's)
+        ~Held() {
+            if (file_ >= 0) (void)flock(file_, LOCK_UN);
+        }
+        explicit operator bool() const { return lock_.owns_lock(); }
+
+    private:
+        std::unique_lock<std::mutex> lock_;
+        int file_ = -1;
+    };
+    // waits for this process's runs; not held while another process makes one
+    Held wait() {
         std::lock_guard<std::mutex> t(turn);
-        return std::unique_lock<std::mutex>(run);
+        return Held(std::unique_lock<std::mutex>(run), *this);
     }
     // not held if a run is under way or waited for
-    std::unique_lock<std::mutex> attempt() {
+    Held attempt() {
         std::unique_lock<std::mutex> t(turn, std::try_to_lock);
-        return t ? std::unique_lock<std::mutex>(run, std::try_to_lock)
-                 : std::unique_lock<std::mutex>();
+        return t ? Held(std::unique_lock<std::mutex>(run, std::try_to_lock), *this) : Held();
+    }
+
+private:
+    // The lock file, open; -1 if it cannot be had (then a run that meets another
+    // process's gives up).  run is held.
+    int file() {
+        if (fd < 0 && !path.empty()) {
+            // (an existing file first: where it is another user's, O_CREAT may
+            // be refused)
+            fd = open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);
+            if (fd < 0) fd = open(path.c_str(), O_RDONLY | O_CREAT | O_CLOEXEC | O_NOFOLLOW, 0444);
+            if (fd < 0) path.clear();
+        }
+        return fd;
     }
 } g_resident[kMaxDevices];
 // host words of a context's resident runs in flight together
@@ -774,8 +823,8 @@ int resident_workspace(seis_model *m, Args &T, int nw, int flag) {
 
 // Makes a resident run on the compute stream and waits for it: launch(T, err)
 // launches it with T's workspace pointers set.  nw: exchange words per cell.
-// *done: 1 if the run was made, 0 if it gave up (the model's state is as before
-// and the caller makes the steps with the step kernels).  ms: device time, if
+// *done: 1 if the run was made, 0 if it gave up or another process makes one (the
+// model's state is as before and the caller makes the steps with the step kernels).  ms: device time, if
 // wanted.
 template <typename Args, typename F>
 int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launch) {
@@ -783,8 +832,9 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     seis_ctx *ctx = m->ctx;
     seis_ctx::Resident &R = ctx->resident;
     hipStream_t st = ctx->stream;
-    const auto lock = g_resident[ctx->device].wait();
     *done = 0;
+    const auto lock = g_resident[ctx->device].wait();
+    if (!lock) return 0;
     if (resident_workspace(m, T, nw, 0)) return 1;
     // (events 0 and 1 time the caller's loop)
     hipEvent_t e0 = pool_event(m, 2), e1 = pool_event(m, 3);
@@ -1162,6 +1212,13 @@ int seis_ctx_create(int device_ordinal, seis_ctx **out) {
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device_ordinal) ==
             hipSuccess)
         ctx->resident.ncu = ncu;
+    if (device_ordinal < kMaxDevices)
+        std::call_once(g_resident[device_ordinal].named, [&] {
+            char pci[32] = "";
+            if (hipDeviceGetPCIBusId(pci, sizeof(pci), device_ordinal) == hipSuccess)
+                g_resident[device_ordinal].path =
+                    std::string("/tmp/seiscl_amd-resident-") + pci + ".lock";
+        });
     *out = ctx.release();
     return 0;
 }
@@ -3568,7 +3625,7 @@ int seis_batch_step(seis_batch *b, int nsteps) {
     std::vector<int> live, resident, left;
     for (int i = 0; i < b->max_slots; ++i)
         if (b->model[i] && b->t[i] < b->tmax[i]) live.push_back(i);
-    std::unique_lock<std::mutex> lock;
+    ResidentLock::Held lock;
     if (b->ctx->resident.open()) lock = g_resident[b->ctx->device].attempt();
     if (lock) {
         std::vector<int> passes;

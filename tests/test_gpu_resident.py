@@ -280,6 +280,46 @@ def test_run_longer_than_the_wait(gpu_ctx, monkeypatch, case):
         assert np.abs(b[-100:]).max() > 0 and np.array_equal(a, b)
 
 
+def test_no_run_beside_another_process(gpu_ctx):
+    """While another process (here: another open file) holds the GPU's lock file,
+    forward, gradient and batch steps are made by the step kernels."""
+    import fcntl
+    import glob
+    from seiscl_amd import Model
+    from seiscl_amd.engine import Batch
+    csts, params, (sp, s, rp) = _shot(dict(ND=2, FDORDER=4, N=(113, 140)))
+    shot = (sp, s, rp[:, :90])
+    m, b = Model(gpu_ctx, params, **csts), Batch(gpu_ctx, 2)
+
+    def run():
+        g, f = _gradient(m, shot)
+        out = m.forward(*shot)
+        m.bind_shot(*shot)
+        slot = b.add(m)
+        b.step(NT)
+        last = m.read_shot()
+        b.remove(slot)
+        return list(g.values()) + f + out + last
+
+    with Runs(gpu_ctx) as free:
+        want = run()
+    locks = [open(p) for p in glob.glob("/tmp/seiscl_amd-resident-*.lock")]
+    for f in locks:
+        fcntl.flock(f, fcntl.LOCK_EX | fcntl.LOCK_NB)
+    with Runs(gpu_ctx) as held:
+        got = run()
+    for f in locks:
+        f.close()
+    with Runs(gpu_ctx) as again:
+        run()
+    b.close()
+    m.close()
+    assert locks and free.made == again.made == (3, 1)
+    assert held.made == (0, 0) and free.gave_up == held.gave_up == again.gave_up == (0, 0)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+
+
 @pytest.mark.parametrize("L", [0, 2])
 def test_runs_beside_another_context(gpu_ctx, L):
     """Resident runs on grids with blocks of halo cells, beside the kernels of a
