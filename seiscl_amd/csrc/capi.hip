@@ -821,10 +821,18 @@ int resident_workspace(seis_model *m, Args &T, int nw, int flag) {
     return 0;
 }
 
+// A run that could not be started counts as one that gave up.
+void resident_lost(seis_ctx::Resident &R, bool adjoint) {
+    (void)hipGetLastError();
+    g_err.clear();
+    R.count(adjoint, false);
+}
+
 // Makes a resident run on the compute stream and waits for it: launch(T, err)
 // launches it with T's workspace pointers set.  nw: exchange words per cell.
-// *done: 1 if the run was made, 0 if it gave up or another process makes one (the
-// model's state is as before and the caller makes the steps with the step kernels).  ms: device time, if
+// *done: 1 if the run was made, 0 if it gave up, found no memory for its words, or
+// another process makes one (the model's state is as before and the caller makes
+// the steps with the step kernels, which need none of it).  ms: device time, if
 // wanted.
 template <typename Args, typename F>
 int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launch) {
@@ -835,15 +843,17 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     *done = 0;
     const auto lock = g_resident[ctx->device].wait();
     if (!lock) return 0;
-    if (resident_workspace(m, T, nw, 0)) return 1;
+    if (resident_workspace(m, T, nw, 0)) {
+        resident_lost(R, adjoint);
+        return 0;
+    }
     // (events 0 and 1 time the caller's loop)
     hipEvent_t e0 = pool_event(m, 2), e1 = pool_event(m, 3);
     if (!e0 || !e1) return fail("hipEventCreate failed");
     HIP_TRY(hipEventRecord(e0, st));
     int e = 0;
     if (!launch(T, &e) || e != hipSuccess) {
-        (void)hipGetLastError();
-        R.count(adjoint, false);
+        resident_lost(R, adjoint);
         return 0;
     }
     HIP_TRY(hipEventRecord(e1, st));
@@ -1652,7 +1662,18 @@ int seis_shot_read_nt(seis_model *m, float *out) {
     const float *src = m->shot.out;
     void *p = nullptr;
     if (nout > 1 || dbl) {
-        if (m->ctx->alloc(n * 4, &p, st)) return 1;
+        if (m->ctx->alloc(n * 4, &p, st)) {
+            // no device memory for the other layout: turned round on the host
+            (void)hipGetLastError();
+            std::vector<float> h(n);
+            if (shot_read(m, h.data(), nullptr)) return 1;
+            for (size_t o = 0; o < (size_t)nout; ++o)
+                for (size_t t = 0; t < (size_t)NT; ++t)
+                    for (size_t r = 0; r < (size_t)nrec; ++r)
+                        out[(o * NT + t) * nrec + r] = h[(o * nrec + r) * NT + t];
+            g_err.clear();
+            return 0;
+        }
         launch_seis_rows(m->shot.out, dbl, (float *)p, NT, nout, nrec, st);
         src = (const float *)p;
     }
@@ -3246,12 +3267,16 @@ int grad_device(seis_model *m, float *out, float *tau, int model) {
     return 0;
 }
 
-// The same into host memory.
+// The same into host memory; -1: no device memory for it (nothing done).
 int grad_to_host(seis_model *m, float *out, float *tau, int model) {
     const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
     hipStream_t st = m->ctx->stream;
     void *p = nullptr;
-    if (m->ctx->alloc(((out ? 3 : 0) + (tau ? 2 : 0)) * n * 4, &p)) return 1;
+    if (m->ctx->alloc(((out ? 3 : 0) + (tau ? 2 : 0)) * n * 4, &p)) {
+        (void)hipGetLastError();
+        g_err.clear();
+        return -1;
+    }
     float *dout = out ? (float *)p : nullptr, *dtau = tau ? (float *)p + (out ? 3 * n : 0) : nullptr;
     int rc = grad_device(m, dout, dtau, model);
     hipError_t e = hipSuccess;
@@ -3280,19 +3305,22 @@ void to_model_layout(const seis_model *m, const std::vector<float> &in, float *o
 int seis_grad_read(seis_model *m, float *grad) {
     g_err.clear();
     if (grad_check(m, false)) return 1;
-    return grad_on_device(m) ? grad_to_host(m, grad, nullptr, 0) : grad_read_host(m, grad);
+    const int rc = grad_on_device(m) ? grad_to_host(m, grad, nullptr, 0) : -1;
+    return rc < 0 ? grad_read_host(m, grad) : rc;
 }
 
 int seis_grad_read_tau(seis_model *m, float *gtau) {
     g_err.clear();
     if (grad_check(m, true)) return 1;
-    return grad_on_device(m) ? grad_to_host(m, nullptr, gtau, 0) : grad_read_tau_host(m, gtau);
+    const int rc = grad_on_device(m) ? grad_to_host(m, nullptr, gtau, 0) : -1;
+    return rc < 0 ? grad_read_tau_host(m, gtau) : rc;
 }
 
 int seis_grad_read_model(seis_model *m, float *grad, float *gtau) {
     g_err.clear();
     if (grad_check(m, false) || (gtau && grad_check(m, true))) return 1;
-    if (grad_on_device(m)) return grad_to_host(m, grad, gtau, 1);
+    const int rc = grad_on_device(m) ? grad_to_host(m, grad, gtau, 1) : -1;
+    if (rc >= 0) return rc;
     const size_t n = (size_t)m->g.NZ * m->g.NY * m->g.NX;
     std::vector<float> h(3 * n);
     if (grad) {
@@ -3593,7 +3621,9 @@ static void batch_split(const seis_batch *b, const std::vector<int> &live, int n
 static int batch_resident(seis_batch *b, const std::vector<int> &slots, int nsteps,
                           std::vector<int> &left) {
     seis_ctx *ctx = b->ctx;
+    seis_ctx::Resident &R = ctx->resident;
     for (size_t k0 = 0; k0 < slots.size(); k0 += kResidentFlags) {
+        bool started[kResidentFlags] = {};
         const size_t k1 = std::min(slots.size(), k0 + kResidentFlags);
         for (size_t k = k0; k < k1; ++k) {
             const int i = slots[k];
@@ -3601,18 +3631,17 @@ static int batch_resident(seis_batch *b, const std::vector<int> &slots, int nste
             Resident2D T = resident_args(m, b->t[i], std::min(nsteps, b->tmax[i] - b->t[i]));
             T.s = b->host_slots[i].shot;
             const int flag = (int)(k - k0);
-            if (resident_workspace(m, T, resident_words(m), flag)) return 1;
             int e = 0;
-            if (!launch_resident2d(T, m->nd_case, ctx->resident.ncu, ctx->stream, &e) ||
-                e != hipSuccess) {
-                (void)hipGetLastError();
-                ctx->resident.failed[flag] = 1;
-            }
+            started[flag] = !resident_workspace(m, T, resident_words(m), flag) &&
+                            launch_resident2d(T, m->nd_case, R.ncu, ctx->stream, &e) &&
+                            e == hipSuccess;
+            if (!started[flag]) resident_lost(R, false);
         }
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         for (size_t k = k0; k < k1; ++k) {
-            const bool done = !((volatile int *)ctx->resident.failed)[k - k0];
-            ctx->resident.count(false, done);
+            const size_t flag = k - k0;
+            const bool done = started[flag] && !((volatile int *)R.failed)[flag];
+            if (started[flag]) R.count(false, done);
             if (!done) left.push_back(slots[k]);
         }
     }
