@@ -42,7 +42,7 @@ template <int H, int L, int NW, int N>
 __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
     constexpr int RZ = 64 + 2 * H, RX = NW * N + 2 * H, FS = RX * RZ;
     constexpr bool BACK = L == 0;               // the forward run is run backwards
-    constexpr int NF = BACK ? 10 : 5, NE = BACK ? 4 : 2;
+    constexpr int NF = BACK ? 10 : 5, NE = resident_adj_values(L);
     constexpr int NP = 8, NC = L ? 8 : 5, LS = L > 0 ? L : 1;
     constexpr int MR = (rim_cells(H, RX - 4 * H, RZ - 4 * H) + 64 * NW - 1) / (64 * NW);
     constexpr int NO = 6;                       // outputs of a receiver
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
         int x0 = x0_, z = z_;
         asm volatile("" : "+s"(x0), "+v"(z));
         const unsigned tag = k + 1;
-        Word *X = a.xch + (size_t)(tag & 1) * nwords<NE>() * g.nfield;
+        Word *X = a.xch + (size_t)(tag & 1) * resident_nwords(NE) * g.nfield;
         const bool last = k + 1 == a.nsteps;
         // 1. adjoint sources (the forward run's were taken out after the exchange)
         if (recs) {

@@ -863,9 +863,9 @@ int resident_run(seis_model *m, Args &T, int nw, int *done, float *ms, F &&launc
     if (ms) HIP_TRY(hipEventElapsedTime(ms, e0, e1));
     return 0;
 }
-int resident_words(const seis_model *m) { return m->nd_case == 22 ? 2 : 4; }
+int forward_words(const seis_model *m) { return resident_words(resident_values(m->nd_case == 22)); }
 int resident_forward(seis_model *m, Resident2D &T, int *done, float *ms = nullptr) {
-    return resident_run(m, T, resident_words(m), done, ms, [&](Resident2D &A, int *e) {
+    return resident_run(m, T, forward_words(m), done, ms, [&](Resident2D &A, int *e) {
         return launch_resident2d(A, m->nd_case, m->ctx->resident.ncu, m->ctx->stream, e);
     });
 }
@@ -2088,7 +2088,6 @@ static int visco_prepare(seis_model *m) {
 // plan, then the seismograms.
 static int forward_save_visco(seis_model *m, float *out) {
     auto &G = m->grad;
-    const seis_csts &c = m->c;
     const int tmax = tmax_of(m);
     hipStream_t st = m->ctx->stream;
     if (visco_prepare(m)) return 1;
@@ -2223,7 +2222,7 @@ static int resident_adjoint(seis_model *m, const AdjArgs<R> &A, int t1, int n, i
             launch_surface_adj(A.r, (R *)G.stmp, m->nd_case, c.gradfix & FIX_SURF_SYY, st);
             *surface = true;
         }
-        return resident_run(m, T, c.L ? 4 : 6, done, nullptr, [&](ResidentAdj2D &B, int *e) {
+        return resident_run(m, T, resident_words(resident_adj_values(c.L)), done, nullptr, [&](ResidentAdj2D &B, int *e) {
             return launch_resident_adj2d(B, c.L, ncu, st, e);
         });
     }
@@ -3632,7 +3631,7 @@ static int batch_resident(seis_batch *b, const std::vector<int> &slots, int nste
             T.s = b->host_slots[i].shot;
             const int flag = (int)(k - k0);
             int e = 0;
-            started[flag] = !resident_workspace(m, T, resident_words(m), flag) &&
+            started[flag] = !resident_workspace(m, T, forward_words(m), flag) &&
                             launch_resident2d(T, m->nd_case, R.ncu, ctx->stream, &e) &&
                             e == hipSuccess;
             if (!started[flag]) resident_lost(R, false);

@@ -79,7 +79,8 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     // the region: 64 + 2H rows of z, NW N + 2H columns
     constexpr int RZ = 64 + 2 * H, RX = NW * N + 2 * H, NF = ACOUSTIC ? 3 : 5, FS = RX * RZ;
     constexpr int NP = ACOUSTIC ? 4 : 8, HP = NP / 4, NC = ACOUSTIC ? 3 : L ? 8 : 5;
-    constexpr int LS = L > 0 ? L : 1, NE = NF - 2;   // NE: exchanged fields
+    constexpr int LS = L > 0 ? L : 1;
+    constexpr int NE = resident_values(ACOUSTIC);   // exchanged fields, the last of NF
     // rim cells per thread
     constexpr int MR = (rim_cells(H, RX - 4 * H, RZ - 4 * H) + 64 * NW - 1) / (64 * NW);
     static_assert(RX * RZ <= 8192, "rlist packing");
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
         int x0 = x0_, z = z_;
         asm volatile("" : "+s"(x0), "+v"(z));
         const unsigned tag = k + 1;
-        Word *X = a.xch + (size_t)(tag & 1) * nwords<NE>() * g.nfield;
+        Word *X = a.xch + (size_t)(tag & 1) * resident_nwords(NE) * g.nfield;
         const bool last = k + 1 == a.nsteps;
         if (ns) {
             if (w == 0) {

@@ -72,8 +72,6 @@ __device__ __forceinline__ Word get_word(const Word *p) {
 // The words of one cell: NE exchanged values (1, 2, 3 or 4) and the number of
 // their step (tag > 0), 32 bits of it beside one value, 16 bits otherwise.
 template <int NE>
-constexpr int nwords() { return NE == 1 ? 1 : NE == 4 ? 3 : 2; }
-template <int NE>
 __device__ __forceinline__ void put_cell(Word *X, long plane, long i, const float *v, unsigned tag) {
     if constexpr (NE <= 2) {
 #pragma unroll
@@ -90,13 +88,13 @@ __device__ __forceinline__ void put_cell(Word *X, long plane, long i, const floa
 template <int NE>
 __device__ __forceinline__ void get_cell(const Word *X, long plane, long i, Word *w) {
 #pragma unroll
-    for (int q = 0; q < nwords<NE>(); ++q) w[q] = get_word(X + q * plane + i);
+    for (int q = 0; q < resident_nwords(NE); ++q) w[q] = get_word(X + q * plane + i);
 }
 template <int NE>
 __device__ __forceinline__ bool cell_ready(const Word *w, unsigned tag) {
     bool r = true;
 #pragma unroll
-    for (int q = 0; q < nwords<NE>(); ++q)
+    for (int q = 0; q < resident_nwords(NE); ++q)
         r = r && (NE <= 2 ? (unsigned)(w[q] >> 32) == tag : (unsigned)(w[q] >> 48) == (tag & 0xffff));
     return r;
 }
@@ -120,7 +118,7 @@ __device__ __forceinline__ void cell_values(const Word *w, float *v) {
 template <int NE, int MR, typename F>
 __device__ __forceinline__ bool take_rim(const Word *X, long plane, unsigned tag,
                                          long long patience, const int *ri, F &&put) {
-    Word v[MR][nwords<NE>()];
+    Word v[MR][resident_nwords(NE)];
     const long long start = wall_clock64();
     auto take = [&](auto first, auto end) {
         constexpr int E0 = decltype(first)::value, E1 = decltype(end)::value;

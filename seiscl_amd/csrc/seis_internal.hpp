@@ -387,7 +387,15 @@ struct AdjArgs {
 // 2D runs resident on the chip (fd2d_resident.hip): FP32, L <= 2 (acoustic
 // L = 0).
 // ---------------------------------------------------------------------------
-constexpr int kResidentMaxRec = 1024, kResidentMaxSrc = 64, kResidentWords = 6;
+constexpr int kResidentMaxRec = 1024, kResidentMaxSrc = 64;
+// Values that a cell exchanges per step: pressure or three stresses, adjoint
+// velocities (without Maxwell bodies the forward run's as well).
+constexpr int resident_values(bool acoustic) { return acoustic ? 1 : 3; }
+constexpr int resident_adj_values(int L) { return L ? 2 : 4; }
+// 64-bit words of that many values with the number of their step, and of a cell's
+// two buffers.
+constexpr int resident_nwords(int values) { return values == 1 ? 1 : values == 4 ? 3 : 2; }
+constexpr int resident_words(int values) { return 2 * resident_nwords(values); }
 struct Resident2D {
     Layout g;
     float hc[7];
@@ -411,7 +419,7 @@ struct Resident2D {
     float *bnd;
     Shell sh;
     float *hist;
-    // exchange words (at most kResidentWords per cell), zero; sync[2], zero: blocks
+    // exchange words (resident_words per cell), zero; sync[2], zero: blocks
     // done, the run's state; failed (host memory): set to 1 by a run that gave
     // up
     unsigned long long *xch;
