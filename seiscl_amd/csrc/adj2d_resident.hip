@@ -52,9 +52,9 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
     __shared__ int rlist[kResidentMaxRec];
     __shared__ float xprof[6 * (kMaxNab + 1)];
     __shared__ float top[5][RX];                // free surface: M, mu, then hx, hz, ts
-    __shared__ int scell[kResidentMaxSrc], stype[kResidentMaxSrc];
+    __shared__ int scell[kResidentMaxSrc], sfield[kResidentMaxSrc];
     __shared__ float samp[kResidentMaxSrc];
-    __shared__ int rcount, dead, verdict;
+    __shared__ int rcount, dead, verdict, pulse;
 
     unsigned tile;
     xcd_tile(a.ntile, tile);
@@ -76,6 +76,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
     if (tid == 0) {
         rcount = 0;
         dead = 0;
+        pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
     }
     float *F = lds + (H + w * N) * RZ + H + lane;
     float co[NC][N], ps[NP][N], mv[3 * LS][N];
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
             if (here) {
                 const int k = __popcll(mask & ((1ull << lane) - 1));
                 scell[k] = sx * RZ + sz;
-                stype[k] = a.s.src_type[lane];
+                sfield[k] = source_field<false>(a.s.src_type[lane]);
                 samp[k] = __int_as_float(lane);
             }
             __builtin_amdgcn_wave_barrier();
@@ -293,11 +294,10 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
                 __builtin_amdgcn_wave_barrier();
                 if (lane == 0)
                     for (int q = 0; q < ns; ++q) {
-                        const int c = scell[q], type = stype[q];
+                        const int c = scell[q], f = sfield[q];
                         const float amp = -1.0f * (a.DT * samp[q]);
-                        if (type == 0) lds[5 * FS + c] = lds[5 * FS + c] + amp;
-                        else if (type == 2) lds[6 * FS + c] = lds[6 * FS + c] + amp;
-                        else if (type == 1 || type == 3 || type == 100)
+                        if (f >= 0) lds[(5 + f) * FS + c] = lds[(5 + f) * FS + c] + amp;
+                        else if (f == kSourceNormal)
                             for (int e = 7; e < 9; ++e)
                                 lds[e * FS + c] =
                                     (float)((double)lds[e * FS + c] + (double)amp / 2.0);
@@ -619,11 +619,9 @@ __global__ __launch_bounds__(64 * NW) void k_resident_adj2d(ResidentAdj2D a) {
         __syncthreads();
         sources_out(a.t1 - a.nsteps + 1);
     }
-    if (tid == 0) {
-        const int pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
+    if (tid == 0)
         verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience,
                         pulse < 0 ? nullptr : a.xch + pulse);
-    }
     __syncthreads();
     if (verdict != 1) return;
 

@@ -87,9 +87,9 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     __shared__ float lds[NF * FS];
     __shared__ int rlist[kResidentMaxRec];             // receiver << 13 | cell
     __shared__ float xprof[6 * (kMaxNab + 1)];
-    __shared__ int scell[kResidentMaxSrc], stype[kResidentMaxSrc];
+    __shared__ int scell[kResidentMaxSrc], sfield[kResidentMaxSrc];
     __shared__ float samp[kResidentMaxSrc];
-    __shared__ int rcount, dead, verdict;
+    __shared__ int rcount, dead, verdict, pulse;
 
     unsigned tile;
     xcd_tile(a.ntile, tile);
@@ -110,6 +110,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     if (tid == 0) {
         rcount = 0;
         dead = 0;
+        pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
     }
     float *F = lds + (H + w * N) * RZ + H + lane;   // the lane's first cell of field 0
     float co[NC][N], ps[NP][N], mv[3 * LS][N];
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
             if (here) {
                 const int k = __popcll(mask & ((1ull << lane) - 1));
                 scell[k] = sx * RZ + sz;
-                stype[k] = a.s.src_type[lane];
+                sfield[k] = source_field<ACOUSTIC>(a.s.src_type[lane]);
                 samp[k] = __int_as_float(lane);
             }
             __builtin_amdgcn_wave_barrier();
@@ -251,23 +252,17 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
                 if (lane == 0) {
                     float *B = lds;
                     for (int q = 0; q < ns; ++q) {
-                        const int c = scell[q], type = stype[q];
+                        const int c = scell[q], f = sfield[q];
                         const float amp = a.DT * samp[q];
-                        int f = -1;
-                        if (type == 0) f = 0;
-                        else if (type == 2) f = 1;
-                        else if (type != 1 && type != 3 && type != 100) continue;
-                        else if (ACOUSTIC) f = type == 1 ? -1 : 2;
-                        // (as sources_body: a y force finds no vy and goes to the
-                        // stresses)
                         if (f >= 0) {
                             B[f * FS + c] = B[f * FS + c] + amp;
                             continue;
                         }
                         if constexpr (!ACOUSTIC)
-                            for (int e = 2; e < 4; ++e)
-                                B[e * FS + c] =
-                                    (float)((double)B[e * FS + c] + (double)amp / 2.0);
+                            if (f == kSourceNormal)
+                                for (int e = 2; e < 4; ++e)
+                                    B[e * FS + c] =
+                                        (float)((double)B[e * FS + c] + (double)amp / 2.0);
                     }
                 }
             }
@@ -532,11 +527,9 @@ __global__ __launch_bounds__(64 * NW) void k_resident2d(Resident2D a) {
     }
 
     // every block's last step is made, or the run has failed
-    if (tid == 0) {
-        const int pulse = pulse_cell<H>(g, CZ, CX, rz0, rx0);
+    if (tid == 0)
         verdict = agree(a.sync, a.failed, (int)a.ntile, dead, a.patience,
                         pulse < 0 ? nullptr : a.xch + pulse);
-    }
     __syncthreads();
     if (verdict != 1) return;
 

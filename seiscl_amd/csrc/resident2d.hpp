@@ -61,6 +61,18 @@ __device__ __forceinline__ void pmlh(float &d, float &psi, const Prof &p) {
     d = d / p.Kh + psi;
 }
 
+// The field a source of a type feeds: 0 vx, 1 vz, 2 p, the normal stresses, or none.
+// A y force has no vy to feed and goes to the normal stresses, as in the step
+// kernels (sources_body).
+constexpr int kSourceNormal = -1, kSourceNone = -2;
+template <bool ACOUSTIC>
+__device__ __forceinline__ int source_field(int type) {
+    if (type == 0) return 0;
+    if (type == 2) return 1;
+    if (type == 3 || type == 100) return ACOUSTIC ? 2 : kSourceNormal;
+    return type == 1 && !ACOUSTIC ? kSourceNormal : kSourceNone;
+}
+
 using Word = unsigned long long;
 __device__ __forceinline__ void put_word(Word *p, Word v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
