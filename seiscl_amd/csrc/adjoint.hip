@@ -187,11 +187,13 @@ __device__ __forceinline__ void taper_apply(const FDArgs<R> &a, int z, int y, in
 // lane -> cell, z fastest; 2D uses y = 0.  In 3D the tiles go on along y, or along
 // x within slabs of ABY rows, dealt to the XCDs in turn where their number allows
 // it (fd3d.hip).  Along y, the 2H + 1 planes that the x-differences of NF fields
-// reach pass through an XCD's L2 whole; from 2.25 MB on (half of it) that is
-// slower.  us, stress and velocity step, along y -> along x: 224 x 192 x 208 elastic
-// 394, 312 -> 374, 293 (7.5 MB); 120 x 128 x 136 96, 75 -> 90, 71 (2.5 MB); L = 2 in
-// half precision 224 x 192 x 208 523, 187 -> 503, 172 (3.8 MB), 150 x 130 x 144 182, 67
-// -> 188, 68.5 (2.1 MB).
+// reach pass through an XCD's L2 (4 MB) whole, among the step's other arrays; once
+// they take half of it or so, that is slower.  The line of 2.25 MiB (2.4 MB) lies
+// between the sizes measured on either side of it.  us, stress and velocity step,
+// along y -> along x: 224 x 192 x 208 elastic 394, 312 -> 374, 293 (7.5 MB);
+// 120 x 128 x 136 96, 75 -> 90, 71 (2.5 MB); L = 2 in half precision
+// 224 x 192 x 208 523, 187 -> 503, 172 (3.8 MB), 150 x 130 x 144 182, 67 -> 188, 68.5
+// (2.1 MB).
 template <typename R, int NF>
 __device__ __forceinline__ bool adj_cell(const Layout &g, int nbz, unsigned nb, int &z, int &y,
                                          int &x) {

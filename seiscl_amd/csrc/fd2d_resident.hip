@@ -48,12 +48,14 @@
 // cells share a window of N + 2H - 1 values, and what depends on x alone is
 // uniform.  The outer H cells of the region have no lane; they are only read.
 //
-// The domain is the padded grid, [-H, N + H) per axis: halo cells are loaded,
-// exchanged and stored like the others and never updated, except for the image
+// The domain is the padded grid, [-H, N + H) per axis: halo cells are loaded
+// and stored like the others, and not updated or exchanged, except for the image
 // rows of the free surface.
 //
 // What bounds a step is the exchange (a store and a load past the L2s, 1.5-2 us)
-// and, from about 1000 cells per CU on, the arithmetic.  Measured on MI355X, us
+// and, from about 1000 cells per CU on, the tile's arithmetic and LDS reads with
+// the barriers between them (at 2100 and 3500 cells per CU the VALUs are busy 44
+// and 41 % of the time, the LDS 31 and 38 %).  Measured on MI355X, us
 // per step, step kernels (replayed graphs) -> this kernel:
 //                     100 x 100    200 x 400    433 x 1217   600 x 1500
 //   elastic FD4       9.5 -> 2.6   9.8 -> 2.9   13.3 -> 6.4  19.9 -> 13.1

@@ -120,9 +120,10 @@ def serve_batched(ctx: Context, requests, max_slots: int = 48, hbm_budget: float
     """Continuous batching.  Set-up threads (setup_threads of them) build
     each admitted request's model (host transforms, uploads on the context's
     transfer stream) while the GPU steps the batch; the main loop moves ready
-    models into free slots, queues the next steps, and only then copies back
-    the jobs that finished in the previous steps, so the GPU always has work
-    queued.  Gradient requests and modeling requests outside the batch
+    models into free slots, makes the next steps, and only then copies back
+    the jobs that finished in the previous steps.  Steps of the batch kernels
+    are queued, so that the GPU works meanwhile; resident runs are waited for
+    (seis_batch_step).  Gradient requests and modeling requests outside the batch
     kernels go, in arrival order, to a worker thread that runs them one at a
     time on a second context (run_alone), beside the batch.
 
